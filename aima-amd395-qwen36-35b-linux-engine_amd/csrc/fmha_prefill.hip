@@ -10,11 +10,16 @@
 //   j <= i + kv_tokens - q_tokens) when kv_tokens > q_tokens.
 //
 // Kernel plan (MFMA-bound, 16384 flop per unmasked (q,k) pair):
-//  * workgroup = 8 waves = 256 query rows of one head; wave = 32 rows; one
-//    workgroup per CU (two waves per SIMD) shares each staged K/V tile
-//    among 256 rows (measured 5-7% faster than two 4-wave workgroups per
-//    CU, which stage every tile twice).  Short square prompts (fewer than
-//    256 such workgroups) use 4- or 2-wave workgroups (128 or 64 rows).
+//  * workgroup = 8 waves = 256 query rows = 32 tokens x the 8 query heads of
+//    one KV head (row r: token r / 8, head r % 8 of the group); wave = 32
+//    rows; one workgroup per CU (two waves per SIMD) shares each staged K/V
+//    tile among 256 rows (measured 5-7% faster than two 4-wave workgroups per
+//    CU, which stage every tile twice).  With the heads of the group in the
+//    rows a tile spans 32 tokens instead of 256, so a short turn fills its
+//    tiles (93 tokens: 3 tiles per KV head, all but 24 of 768 rows live, where
+//    256-token tiles of 8 heads left 163 of every 256 rows dead) and only a
+//    tile's last 32 keys are masked.  Fewer than 32 tokens use 4- or 2-wave
+//    workgroups (16 or 8 tokens).
 //  * per 32-key tile: K and V are staged in LDS (padded row-pair blocks, so
 //    every LDS address is a per-lane base plus an immediate); S^T = K Q^T on
 //    v_mfma_f32_32x32x16_bf16 (A = K from LDS, B = Q^T held in registers for
@@ -31,12 +36,13 @@
 //  * no per-tile row max: the reference max is the first tile's, raised
 //    (with a rescale of O) only when a tile's probabilities would exceed
 //    2^20, which the per-lane probability sum detects.
-//  * blockIdx -> (KV head, query head, query tile) is XCD-aware: the 8 XCDs
+//  * blockIdx -> (KV head, query tile) is XCD-aware: the 8 XCDs
 //    receive workgroups round-robin, so XCDs 0-3 serve KV head 0 and 4-7 KV
 //    head 1 (their L2s then hold one head's K/V), and every XCD issues its
 //    heaviest (latest) causal tiles first.
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace q36 {
@@ -66,11 +72,11 @@ constexpr int kFmLdsGated = kFmLds + kFmGateLds;      // 133632
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// Split-K partials (kSplit): workgroup (q tile, chunk, head) writes its
+// Split-K partials (kSplit): workgroup (q tile, chunk, KV head) writes its
 // unnormalised O rows and (m, l) for keys [chunk * chunk_keys, +chunk_keys).
 struct SplitArgs {
-  float* o;             // [tile][chunk][head][256 rows][256]
-  float* ml;            // [tile][chunk][head][256 rows][2]
+  float* o;             // [tile][chunk][kv head][rows][256]
+  float* ml;            // [tile][chunk][kv head][rows][2]
   unsigned chunk_keys;  // multiple of 32
   unsigned n_chunks;
 };
@@ -85,44 +91,50 @@ struct GateArgs {
 };
 
 template <int kFmWaves, bool kSplit, bool kGate = false>
-__global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
+__global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k,
     const bf16* __restrict__ v, float* __restrict__ out, unsigned q_tokens,
     unsigned kv_tokens, unsigned n_qtiles, SplitArgs sp, GateArgs ga) {
   static_assert(!(kSplit && kGate), "split partials are gated by the combine");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int kFmRows = kFmWaves * kFmRowsPerWave;
+  constexpr unsigned kTok = kFmRows / kGroup;          // tokens per tile
   constexpr int kFmLoadsPerWave = 16 / kFmWaves;       // 16 row-pair blocks per tile
 
-  // XCD-aware tile mapping (see header); split: (tile, chunk, head).
-  const unsigned b = blockIdx.x;
-  int kvh, head;
+  // XCD-aware tile mapping (see header).  Split: the (chunk, tile) items of a
+  // KV head, chunk by chunk and heaviest tile first, are dealt to its four
+  // XCDs in turn (contiguous ranges, so that a chunk's rows go to one L2,
+  // measured no faster: 1000 rows over 4096 96 us against 90).
+  const unsigned b = blockIdx.x, n = b >> 3, x4 = b & 3;
+  const int kvh = (b >> 2) & 1;
   unsigned qtile, chunk = 0;
   if constexpr (kSplit) {
-    head = (int)(b % kHq);
-    kvh = head / kGroup;
-    qtile = (b / kHq) / sp.n_chunks;
-    chunk = (b / kHq) % sp.n_chunks;
+    const unsigned i = 4 * n + x4;
+    if (i >= n_qtiles * sp.n_chunks) return;
+    chunk = i / n_qtiles;
+    qtile = n_qtiles - 1 - i % n_qtiles;
   } else {
-    const unsigned xcd = b & 7u, n = b >> 3;
-    kvh = xcd >> 2;
-    head = kvh * kGroup + (xcd & 3) * 2 + (n & 1);
-    qtile = n_qtiles - 1 - (n >> 1);
+    if (4 * n + x4 >= n_qtiles) return;
+    qtile = n_qtiles - 1 - (4 * n + x4);
   }
-  const unsigned q0 = qtile * kFmRows;
+  const unsigned tok0 = qtile * kTok;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lj = lane & 31;     // MFMA column (query row within the wave)
   const int lg = lane >> 5;     // k-half
   const unsigned off = kv_tokens - q_tokens;   // bottom-right shift
-  const unsigned row = q0 + wave * kFmRowsPerWave + lj;   // this lane's query
-  const bool row_valid = row < q_tokens;
-  const unsigned row_lim = (row_valid ? row : q_tokens - 1) + off;  // last key
-  const unsigned wave_first = q0 + wave * kFmRowsPerWave;
+  // this lane's query: token `tok`, query head `head`
+  const unsigned row = wave * kFmRowsPerWave + lj;   // row of the tile
+  const unsigned tok = tok0 + row / kGroup;
+  const int head = kvh * kGroup + (int)(row % kGroup);
+  const bool row_valid = tok < q_tokens;
+  const unsigned row_lim = (row_valid ? tok : q_tokens - 1) + off;  // last key
+  const unsigned wave_first = tok0 + wave * (kFmRowsPerWave / kGroup);   // first token
+  const bool wave_live = wave_first < q_tokens;
   const unsigned wave_lim =
-      min(wave_first + kFmRowsPerWave - 1, q_tokens - 1) + off;
-  const unsigned kv_end = min(kv_tokens, min(q0 + kFmRows, q_tokens) + off);
+      min(wave_first + kFmRowsPerWave / kGroup - 1, q_tokens - 1) + off;
+  const unsigned kv_end = min(kv_tokens, min(tok0 + kTok, q_tokens) + off);
   // key range of this workgroup: whole rows, or one chunk of them
   const unsigned kv_first = kSplit ? chunk * sp.chunk_keys : 0u;
   const unsigned kv_stop = kSplit ? min(kv_end, kv_first + sp.chunk_keys) : kv_end;
@@ -131,7 +143,7 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
   // Q^T operand: step s covers dims s*16 + 8*lg .. +8 of this lane's row.
   bf16x8 qf[16];
   {
-    const bf16* qp = q + (size_t)row * kQDim + head * kD + 8 * lg;
+    const bf16* qp = q + (size_t)tok * kQDim + head * kD + 8 * lg;
 #pragma unroll
     for (int s = 0; s < 16; ++s)
       qf[s] = row_valid ? *reinterpret_cast<const bf16x8*>(qp + s * 16)
@@ -158,16 +170,17 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
   // (row-major [256 rows][256 B]), fetched now so they are resident when the
   // epilogue starts; rows past the end read as zeros.
   if constexpr (kGate) {
-    const unsigned rows_here = min(q_tokens - q0, (unsigned)kFmRows);
+    const unsigned toks_here = min(q_tokens - tok0, kTok);
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16*>(ga.gate) + (size_t)q0 * ga.gate_stride + head * 2 * kD + kD, 0,
-        (int)(rows_here * ga.gate_stride * 2), 0x00020000);
+        const_cast<bf16*>(ga.gate) + (size_t)tok0 * ga.gate_stride, 0,
+        (int)(toks_here * ga.gate_stride * 2), 0x00020000);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int r0 = wave * kFmRowsPerWave + 4 * j;
+      const int r0 = wave * kFmRowsPerWave + 4 * j, r = r0 + (lane >> 4);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           grs, (lds_void*)(lds + kFmLds + r0 * 256), 16,
-          (int)(((r0 + (lane >> 4)) * ga.gate_stride) * 2 + (lane & 15) * 16), 0, 0, 0);
+          (int)((r / kGroup) * ga.gate_stride * 2 +
+                ((kvh * kGroup + r % kGroup) * 2 * kD + kD) * 2 + (lane & 15) * 16), 0, 0, 0);
     }
   }
   auto fetch = [&](unsigned kv0, int stage) {
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
     __builtin_amdgcn_s_waitcnt(0);   // this wave's fetches of tile t landed
     __syncthreads();                 // ... and every wave's; tile t-1 consumed
     if (t + 1 < n_tiles) fetch(kv0 + kFmKv, stage ^ 1);
-    if (kv0 > wave_lim) continue;    // every key of the tile is masked for us
+    if (kv0 > wave_lim || !wave_live) continue;   // no row of ours sees a key of the tile
     const char* kp = lds + stage * kFmStage + kbase;
     const char* vp = lds + stage * kFmStage + kKTile + vbase;
 
@@ -308,16 +321,15 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
   l += __shfl_xor(l, 32, 64);
   if constexpr (kSplit) {
     if (!row_valid) return;
-    const size_t item = ((size_t)qtile * sp.n_chunks + chunk) * kHq + head;
-    const unsigned r = row - q0;
-    float* op = sp.o + (item * kFmRows + r) * kD + 4 * lg;
+    const size_t item = ((size_t)qtile * sp.n_chunks + chunk) * kHkv + kvh;
+    float* op = sp.o + (item * kFmRows + row) * kD + 4 * lg;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4)
         *reinterpret_cast<f32x4*>(op + dt * 32 + 8 * r4) =
             f32x4{o[dt][4 * r4], o[dt][4 * r4 + 1], o[dt][4 * r4 + 2], o[dt][4 * r4 + 3]};
-    if (lg == 0) *reinterpret_cast<float2*>(sp.ml + (item * kFmRows + r) * 2) = float2{m, l};
+    if (lg == 0) *reinterpret_cast<float2*>(sp.ml + (item * kFmRows + row) * 2) = float2{m, l};
     return;
   } else {
     // The output leaves through LDS in four rounds of 64 dims: each wave
@@ -326,7 +338,6 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
     // and stores whole 256-byte row segments, instead of 32-byte pieces of
     // 32 rows per store instruction.
     const float inv = row_valid ? 1.0f / l : 0.f;
-    const unsigned wrow0 = q0 + wave * kFmRowsPerWave;
     // gated: rounds 0-1 take their gate values from the LDS prefetch; the
     // register loads of rounds 2-3 are issued now and land behind rounds 0-1
     // (rows past the end read the last row's and are not stored)
@@ -337,10 +348,11 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
       for (int rd = 0; rd < 2; ++rd)
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
-          const unsigned r = min(wrow0 + it * 4 + (lane >> 4), q_tokens - 1);
+          const unsigned r = it * 4 + (lane >> 4);
+          const unsigned t = min(wave_first + r / kGroup, q_tokens - 1);
           gv[rd][it] = *reinterpret_cast<const bf16x4*>(
-              ga.gate + (size_t)r * ga.gate_stride + head * 2 * kD + kD + (rd + 2) * 64 +
-              (lane & 15) * 4);
+              ga.gate + (size_t)t * ga.gate_stride + (kvh * kGroup + r % kGroup) * 2 * kD + kD +
+              (rd + 2) * 64 + (lane & 15) * 4);
         }
     }
     __syncthreads();   // every wave is done with the K/V ring
@@ -365,20 +377,19 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
       for (int it = 0; it < 8; ++it) {
         const int r = it * 4 + (lane >> 4), ch = lane & 15;
         const f32x4 v = *reinterpret_cast<const f32x4*>(stg + r * 256 + ((ch ^ (r & 15)) * 16));
+        const unsigned t = wave_first + r / kGroup;
+        const size_t orow = (size_t)t * kQDim + (kvh * kGroup + r % kGroup) * kD + rd * 64 + ch * 4;
         if constexpr (kGate) {
-          if (wrow0 + r < q_tokens) {
+          if (t < q_tokens) {
             const bf16x4 g4 =
                 rd < 2 ? *reinterpret_cast<const bf16x4*>(lds + kFmLds + (wave * kFmRowsPerWave + r) * 256 +
                                                           rd * 128 + ch * 8)
                        : gv[rd - 2][it];
-            *reinterpret_cast<bf16x4*>(ga.out + (size_t)(wrow0 + r) * kQDim + head * kD +
-                                       rd * 64 + ch * 4) = gate4_bf16_fast(v, g4);
+            *reinterpret_cast<bf16x4*>(ga.out + orow) = gate4_bf16_fast(v, g4);
           }
-        } else if (wrow0 + r < q_tokens) {
+        } else if (t < q_tokens) {
           // nontemporal: the output is not re-read here (459.0 vs 460.0 us at 8K)
-          __builtin_nontemporal_store(
-              v, reinterpret_cast<f32x4*>(out + (size_t)(wrow0 + r) * kQDim + head * kD +
-                                          rd * 64 + ch * 4));
+          __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(out + orow));
         }
       }
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -386,41 +397,48 @@ __global__ __launch_bounds__(64 * kFmWaves, 1) void fmha_prefill_kernel(
   }
 }
 
-// Split-K combine: thread (row, 8 dims) of (q tile, head) merges the live
-// chunks' partials: M = max m_c, L = sum l_c 2^(m_c - M), O = sum O_c 2^(m_c -
-// M) / L (chunks where the row saw no key have l = 0 and weigh nothing).
-// grid = tiles x 16 heads x 16 row groups; block = 512 (16 rows x 32 dims/8).
-// Every (m, l) pair, the first four chunks' O partials and the gate are
-// requested together (indices clamped to the live range, so every load is
-// unconditional and in bounds): one memory round trip for up to four live
-// chunks, where per-chunk loads behind the l > 0 test cost two each.
-constexpr int kCombineMaxChunks = 16;   // split_plan: n_chunks <= 256 / 16
-template <int kMaxC>   // n_chunks <= kMaxC (4 or kCombineMaxChunks)
+// Split-K combine: kG groups of 32 threads (8 dims each) merge the live
+// chunks' partials of one (token, head) row, group g chunks g, g + kG, ...:
+// M = max m_c, L = sum l_c 2^(m_c - M), O = sum O_c 2^(m_c - M) / L (chunks
+// where the row saw no key have l = 0 and weigh nothing), then the groups
+// through LDS, in group order.  block = 512 = 16 / kG rows of 32 kG threads.
+// A group's (m, l) pairs, its first four chunks' O partials and the gate
+// are requested together (indices clamped to the live range, so every load
+// is unconditional and in bounds): one memory round trip for up to four
+// is unconditional and in bounds): one memory round trip for up to four
+// chunks a group, so the launch picks kG for at most four.  The reads bound
+// it: 42 chunks of 93 tokens, 62 MB, 12.9 us (with 8 groups of up to 16
+// chunks the split and combine took 62 us, with 16 of 4 they take 59).
+constexpr int kCombineMaxChunks = 128;   // split_plan's most
+template <int kG, int kMaxC>   // kMaxC: chunks per group at most, a multiple of 4
 __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
     const float* __restrict__ po, const float* __restrict__ pml, float* __restrict__ out,
-    unsigned q_tokens, unsigned kv_tokens, unsigned chunk_keys, unsigned n_chunks,
-    GateArgs ga) {
-  constexpr int kRows = 256;
-  const unsigned rg = blockIdx.x % 16, head = (blockIdx.x / 16) % kHq, qtile = blockIdx.x / (16 * kHq);
-  const unsigned r = rg * 16 + (threadIdx.x >> 5);
-  const unsigned row = qtile * kRows + r;
-  if (row >= q_tokens) return;
+    unsigned q_tokens, unsigned kv_tokens, unsigned tile_toks, unsigned chunk_keys,
+    unsigned n_chunks, GateArgs ga) {
+  constexpr unsigned kRowsHere = 16 / kG;
+  __shared__ __attribute__((aligned(16))) float part[kG > 1 ? 512 : 1][8];
+  __shared__ float2 part_ml[16];
+  const unsigned g = (threadIdx.x >> 5) % kG;
+  const unsigned rid = blockIdx.x * kRowsHere + (threadIdx.x >> 5) / kG;   // token * 16 + head
+  const unsigned tok = rid / kHq, head = rid % kHq, kvh = head / kGroup;
+  const unsigned qtile = tok / tile_toks, rows = tile_toks * kGroup;
+  const unsigned r = (tok - qtile * tile_toks) * kGroup + head % kGroup;   // row of the tile
   const int d0 = 8 * (threadIdx.x & 31);
   const unsigned off = kv_tokens - q_tokens;
-  const unsigned kv_end = min(kv_tokens, min(qtile * kRows + kRows, q_tokens) + off);
+  const unsigned kv_end = min(kv_tokens, min((qtile + 1) * tile_toks, q_tokens) + off);
   const unsigned live = (kv_end + chunk_keys - 1) / chunk_keys;   // 1 .. n_chunks
-  auto item_of = [&](unsigned c) {
-    return ((size_t)qtile * n_chunks + min(c, live - 1)) * kHq + head;
+  auto row_of = [&](unsigned c) {
+    return (((size_t)qtile * n_chunks + min(c, live - 1)) * kHkv + kvh) * rows + r;
   };
   float2 ml[kMaxC];
 #pragma unroll
   for (int c = 0; c < kMaxC; ++c)
-    ml[c] = *reinterpret_cast<const float2*>(pml + (item_of(c) * kRows + r) * 2);
+    ml[c] = *reinterpret_cast<const float2*>(pml + row_of(g + kG * c) * 2);
   f32x4 oa[4], ob[4];
   auto load_o = [&](int c0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const f32x4* src = reinterpret_cast<const f32x4*>(po + (item_of(c0 + j) * kRows + r) * kD + d0);
+      const f32x4* src = reinterpret_cast<const f32x4*>(po + row_of(g + kG * (c0 + j)) * kD + d0);
       oa[j] = src[0];
       ob[j] = src[1];
     }
@@ -428,23 +446,23 @@ __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
   load_o(0);
   // gated: the gate row (any valid address otherwise; the value is unused)
   const bf16* gp = ga.out != nullptr
-                       ? ga.gate + (size_t)row * ga.gate_stride + head * 2 * kD + kD + d0
-                       : reinterpret_cast<const bf16*>(po + (item_of(0) * kRows + r) * kD + d0);
-  const bf16x8 g = *reinterpret_cast<const bf16x8*>(gp);
+                       ? ga.gate + (size_t)tok * ga.gate_stride + head * 2 * kD + kD + d0
+                       : reinterpret_cast<const bf16*>(po + row_of(0) * kD + d0);
+  const bf16x8 gv = *reinterpret_cast<const bf16x8*>(gp);
   __builtin_amdgcn_sched_barrier(0);
   float M = -INFINITY;
 #pragma unroll
   for (int c = 0; c < kMaxC; ++c)
-    if ((unsigned)c < live && ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
+    if (g + kG * c < live && ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
   float L = 0.f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int c0 = 0; c0 < kMaxC; c0 += 4) {
-    if ((unsigned)c0 >= live) break;
+    if (g + kG * c0 >= live) break;
     if (c0 > 0) load_o(c0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float2 m_l = ml[c0 + j];
-      if ((unsigned)(c0 + j) < live && m_l.y > 0.f) {
+      if (g + kG * (c0 + j) < live && m_l.y > 0.f) {
         const float w = __builtin_amdgcn_exp2f(m_l.x - M);
         L += w * m_l.y;
 #pragma unroll
@@ -455,22 +473,50 @@ __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
       }
     }
   }
+  if constexpr (kG > 1) {
+    f32x4* mine = reinterpret_cast<f32x4*>(part[threadIdx.x]);
+    mine[0] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    mine[1] = f32x4{acc[4], acc[5], acc[6], acc[7]};
+    if ((threadIdx.x & 31) == 0) part_ml[threadIdx.x >> 5] = float2{M, L};
+    __syncthreads();
+    if (g != 0) return;
+    float m_all = M;   // key 0's chunk is live: some group has L > 0
+#pragma unroll
+    for (int j = 1; j < kG; ++j) m_all = fmaxf(m_all, part_ml[(threadIdx.x >> 5) + j].x);
+    const float w0 = L > 0.f ? __builtin_amdgcn_exp2f(M - m_all) : 0.f;
+    L *= w0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= w0;
+#pragma unroll
+    for (int j = 1; j < kG; ++j) {
+      const float2 m_l = part_ml[(threadIdx.x >> 5) + j];
+      const float w = m_l.y > 0.f ? __builtin_amdgcn_exp2f(m_l.x - m_all) : 0.f;
+      L += w * m_l.y;
+      const f32x4* src = reinterpret_cast<const f32x4*>(part[threadIdx.x + 32 * j]);
+      const f32x4 a = src[0], b = src[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[e] += w * a[e];
+        acc[4 + e] += w * b[e];
+      }
+    }
+  }
   const float inv = 1.0f / L;
   if (ga.out != nullptr) {   // gated bf16 rows (see GateArgs)
     const bf16x4 lo = gate4_bf16_fast(f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv},
-                                      bf16x4{g[0], g[1], g[2], g[3]});
+                                      bf16x4{gv[0], gv[1], gv[2], gv[3]});
     const bf16x4 hi = gate4_bf16_fast(f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv},
-                                      bf16x4{g[4], g[5], g[6], g[7]});
-    *reinterpret_cast<bf16x8*>(ga.out + (size_t)row * kQDim + head * kD + d0) =
+                                      bf16x4{gv[4], gv[5], gv[6], gv[7]});
+    *reinterpret_cast<bf16x8*>(ga.out + (size_t)tok * kQDim + head * kD + d0) =
         bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return;
   }
-  f32x4* dst = reinterpret_cast<f32x4*>(out + (size_t)row * kQDim + head * kD + d0);
+  f32x4* dst = reinterpret_cast<f32x4*>(out + (size_t)tok * kQDim + head * kD + d0);
   dst[0] = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
   dst[1] = f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
 }
 
-// Split-K scratch: room for kSplitItems (tile, chunk, head) partials of 256
+// Split-K scratch: room for kSplitItems (tile, chunk, KV head) partials of 256
 // rows.  The reference's provider ABI has no workspace argument, so the
 // provider owns one scratch per device (allocated by qrt_ck_fmha_prepare,
 // kept until the process ends: graphs captured with a split launch hold its
@@ -508,40 +554,61 @@ void* provider_scratch_for(hipStream_t stream) {
 std::once_flag g_fm_attr_once;
 hipError_t g_fm_attr_status = hipSuccess;
 
-// Split plan for short prompts: too few 256-row tiles to fill the GPU, so
-// each tile's key range is cut into n chunks (a multiple of 32 keys; a
-// tile's chunks past its last key exit at once).  The chunk count was
-// swept on MI355X (n = 2 .. 16 and unsplit, graph-replayed):
-//  * square prompts (no cached prefix): the best n by 256-row tile count,
-//    kSquareChunks below (T = 256: 23.9 us at n = 2 against 27.7 at 16;
-//    T = 2304 / 2560: 85 / 97 us at n = 3 against 92 / 107 at 2);
-//  * rows over a prefix: about 256 workgroups (n = 256 / (16 tiles));
-//  * from 11 tiles on (T > 2560) the unsplit kernel is faster than any
-//    split that fits the scratch (T = 3072 128 vs 137 us, T = 3840 165 vs
-//    182; 3072 rows over a 4096 prefix 290 vs 327).
+// Split plan for short prompts: too few query tiles to fill the GPU, so each
+// tile's key range is cut into n chunks (a multiple of 32 keys; a tile's
+// chunks past its last key exit at once), and few rows take smaller tiles.
+// Swept on MI355X over 1 .. 8192 tokens, prefixes of 0 .. 64000 and n = 1 ..
+// 128 (graph-replayed, gated):
+//  * rows over a prefix: every tile has about the same work, so n makes about
+//    one workgroup per CU, of at least 96 keys each (93 rows over 24000: n =
+//    32 .. 42 60 us, 16 73, 64 70; 8 over 65000: 33 us at 128, 41 at 64, 50 at
+//    32).  8 waves, whose tiles read K/V least often, from tokens x keys =
+//    1.4 M (256 over 8000: 54 us against 55; 64 over 64000: 86 against 98),
+//    4 waves below (93 over 8000: 34 us against 38), 2 waves below 0.1 M.
+//    Up to 3072 rows two chunks still win (2500 over 4000: 219 us against
+//    299 unsplit; 3500: 339 against 325).
+//  * square prompts: later tiles hold more chunks, 2 tiles (n + 1) / 2 in
+//    all, again about one per CU: n = 4 up to 42 tiles, 3 up to 66, then 2
+//    (2048 tokens: 63 us at n = 3, 68 at 2, 86 at 4; 3072: 105 us at 2, 120
+//    at 4, 134 unsplit) up to 4096 (166 us against 181; 4500: 204 against
+//    200).  8-token tiles up to 360 tokens (256: 16 us against 17), 16-token
+//    tiles up to 960 (768: 29 us against 33; 1000: 37 against 36).
 struct SplitPlan {
-  unsigned n_chunks, chunk_keys, items;
+  unsigned waves, tiles, n_chunks, chunk_keys, items;   // items: (tile, chunk, KV head) partials
 };
 
-constexpr unsigned kSplitMaxTiles = 10;
-constexpr unsigned char kSquareChunks[kSplitMaxTiles + 1] = {0, 2, 8, 6, 4, 4, 3, 3, 2, 3, 3};
+unsigned tile_tokens(unsigned waves) { return waves * kFmRowsPerWave / kGroup; }
 
 SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
-  const unsigned tiles = (q_tokens + 255) / 256;
-  SplitPlan p{1u, kv_tokens, 0u};
-  if (tiles > kSplitMaxTiles) return p;
-  p.n_chunks = kv_tokens - q_tokens < 256u ? kSquareChunks[tiles]
-                                           : (256u + tiles * kHq - 1) / (tiles * kHq);
-  p.chunk_keys = (((kv_tokens + p.n_chunks - 1) / p.n_chunks) + kFmKv - 1) / kFmKv * kFmKv;
-  p.n_chunks = (kv_tokens + p.chunk_keys - 1) / p.chunk_keys;   // after rounding up
-  p.items = tiles * p.n_chunks * kHq;
-  if (p.n_chunks < 2 || p.items > kSplitItems) p = SplitPlan{1u, kv_tokens, 0u};
-  static_assert(256 / kHq <= kCombineMaxChunks, "the combine holds every chunk's (m, l)");
+  SplitPlan p{};
+  p.n_chunks = 1u;
+  p.chunk_keys = kv_tokens;
+  const bool square = kv_tokens - q_tokens < 256u;
+  if (q_tokens > (square ? 4096u : 3072u)) return p;
+  const size_t work = (size_t)q_tokens * kv_tokens;
+  if (square)
+    p.waves = q_tokens <= 360u ? 2u : q_tokens <= 960u ? 4u : 8u;
+  else
+    p.waves = work <= 100000u ? 2u : work <= 1400000u ? 4u : 8u;
+  p.tiles = (q_tokens + tile_tokens(p.waves) - 1) / tile_tokens(p.waves);
+  unsigned n;
+  if (square) {
+    n = p.tiles <= 42u ? 4u : p.tiles <= 66u ? 3u : 2u;
+  } else {
+    n = std::min(128u / p.tiles, kv_tokens / 96u);
+    n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
+  }
+  const unsigned chunk = ((kv_tokens + n - 1) / n + kFmKv - 1) / kFmKv * kFmKv;
+  n = (kv_tokens + chunk - 1) / chunk;   // after rounding up
+  if (n < 2u) return p;
+  p.n_chunks = n;
+  p.chunk_keys = chunk;
+  p.items = p.tiles * n * kHkv;          // at most kSplitItems
   return p;
 }
 
 size_t split_workspace_bytes(const SplitPlan& p) {
-  return p.n_chunks > 1 ? (size_t)p.items * kSplitItemBytes : 0;
+  return p.n_chunks > 1 ? (size_t)p.items * (p.waves * kFmRowsPerWave) * (kD + 2) * sizeof(float) : 0;
 }
 
 bool valid_geometry(const void* q, const void* k, const void* v, const float* out,
@@ -559,7 +626,9 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
     for (const void* f : {reinterpret_cast<const void*>(fmha_prefill_kernel<8, false>),
                           reinterpret_cast<const void*>(fmha_prefill_kernel<4, false>),
                           reinterpret_cast<const void*>(fmha_prefill_kernel<2, false>),
-                          reinterpret_cast<const void*>(fmha_prefill_kernel<8, true>)}) {
+                          reinterpret_cast<const void*>(fmha_prefill_kernel<8, true>),
+                          reinterpret_cast<const void*>(fmha_prefill_kernel<4, true>),
+                          reinterpret_cast<const void*>(fmha_prefill_kernel<2, true>)}) {
       const hipError_t e =
           hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kFmLds);
       if (e != hipSuccess) g_fm_attr_status = e;
@@ -570,45 +639,66 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
     if (e != hipSuccess) g_fm_attr_status = e;
   });
   if (g_fm_attr_status != hipSuccess) return (int)g_fm_attr_status;
-  auto tiles = [&](unsigned rows) { return (q_tokens + rows - 1) / rows; };
   const bf16* qb = static_cast<const bf16*>(q);
   const bf16* kb = static_cast<const bf16*>(k);
   const bf16* vb = static_cast<const bf16*>(v);
-  const SplitArgs none{nullptr, nullptr, 0u, 1u};
   const SplitPlan plan = split_plan(q_tokens, kv_tokens);
   if (plan.n_chunks > 1 && scratch != nullptr) {
     SplitArgs sp;
     sp.o = static_cast<float*>(scratch);
-    sp.ml = sp.o + (size_t)plan.items * 256 * kD;   // (O partials, then (m, l) pairs)
+    sp.ml = sp.o + (size_t)plan.items * (plan.waves * kFmRowsPerWave) * kD;   // after the O partials
     sp.chunk_keys = plan.chunk_keys;
     sp.n_chunks = plan.n_chunks;
-    hipLaunchKernelGGL((fmha_prefill_kernel<8, true>), dim3(plan.items), dim3(512), kFmLds,
-                       stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(256), sp, ga);
-    auto combine = plan.n_chunks <= 4 ? fmha_split_combine_kernel<4>
-                                      : fmha_split_combine_kernel<kCombineMaxChunks>;
-    hipLaunchKernelGGL(combine, dim3(tiles(256) * kHq * 16), dim3(512), 0, stream, sp.o, sp.ml,
-                       out, q_tokens, kv_tokens, plan.chunk_keys, plan.n_chunks, ga);
+    auto split = plan.waves == 8   ? fmha_prefill_kernel<8, true>
+                 : plan.waves == 4 ? fmha_prefill_kernel<4, true>
+                                   : fmha_prefill_kernel<2, true>;
+    hipLaunchKernelGGL(split, dim3(8 * ((plan.tiles * plan.n_chunks + 3) / 4)),
+                       dim3(64 * plan.waves), kFmLds, stream, qb, kb, vb, out, q_tokens, kv_tokens,
+                       plan.tiles, sp, ga);
+    // groups of 32 threads per row: at most 4 chunks (one round trip) a group,
+    // 8 past 64 chunks
+    unsigned groups = 16;
+    auto combine = fmha_split_combine_kernel<16, kCombineMaxChunks / 16>;
+    if (plan.n_chunks <= 4) {
+      groups = 1;
+      combine = fmha_split_combine_kernel<1, 4>;
+    } else if (plan.n_chunks <= 8) {
+      groups = 2;
+      combine = fmha_split_combine_kernel<2, 4>;
+    } else if (plan.n_chunks <= 16) {
+      groups = 4;
+      combine = fmha_split_combine_kernel<4, 4>;
+    } else if (plan.n_chunks <= 32) {
+      groups = 8;
+      combine = fmha_split_combine_kernel<8, 4>;
+    } else if (plan.n_chunks <= 64) {
+      combine = fmha_split_combine_kernel<16, 4>;
+    }
+    hipLaunchKernelGGL(combine, dim3(q_tokens * groups), dim3(512), 0, stream, sp.o, sp.ml,
+                       out, q_tokens, kv_tokens, tile_tokens(plan.waves), plan.chunk_keys,
+                       plan.n_chunks, ga);
     return static_cast<int>(hipGetLastError());
   }
+  const SplitArgs none{nullptr, nullptr, 0u, 1u};
+  auto tiles = [&](unsigned waves) { return (q_tokens + tile_tokens(waves) - 1) / tile_tokens(waves); };
+  auto grid = [&](unsigned waves) { return dim3(8 * ((tiles(waves) + 3) / 4)); };
   if (ga.out != nullptr) {   // gated: 256-row workgroups at every length
-    hipLaunchKernelGGL((fmha_prefill_kernel<8, false, true>), dim3(tiles(256) * kHq), dim3(512),
-                       kFmLdsGated, stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(256), none, ga);
+    hipLaunchKernelGGL((fmha_prefill_kernel<8, false, true>), grid(8), dim3(512),
+                       kFmLdsGated, stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(8), none, ga);
     return static_cast<int>(hipGetLastError());
   }
-  // Query rows per workgroup: 256 (8 waves) when that gives at least 256
-  // workgroups or the rows extend a cached prefix (long rows); short square
-  // prompts use 128 or 64 rows so they still spread over the CUs (measured on
-  // MI355X: T = 1024 51 vs 54 us, T = 2048 96 vs 97-102 us; 8 waves stay best
-  // from T = 4096 and for 1024 rows over a 4096-token prefix).
-  if (tiles(256) * kHq >= 256u || kv_tokens > q_tokens) {
-    hipLaunchKernelGGL((fmha_prefill_kernel<8, false>), dim3(tiles(256) * kHq), dim3(512),
-                       kFmLds, stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(256), none, ga);
-  } else if (tiles(128) * kHq >= 256u) {
-    hipLaunchKernelGGL((fmha_prefill_kernel<4, false>), dim3(tiles(128) * kHq), dim3(256),
-                       kFmLds, stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(128), none, ga);
+  // Rows per workgroup without a split: 256 (8 waves) when that gives at
+  // least 256 workgroups or the rows extend a cached prefix (long rows); short
+  // square prompts use 128 or 64 rows so they still spread over the CUs.
+  if (2 * tiles(8) >= 256u || kv_tokens > q_tokens) {
+    hipLaunchKernelGGL((fmha_prefill_kernel<8, false>), grid(8), dim3(512), kFmLds, stream,
+                       qb, kb, vb, out, q_tokens, kv_tokens, tiles(8), none, ga);
+  } else if (2 * tiles(4) >= 256u) {
+    hipLaunchKernelGGL((fmha_prefill_kernel<4, false>), grid(4), dim3(256), kFmLds, stream,
+                       qb, kb, vb, out, q_tokens, kv_tokens, tiles(4), none, ga);
   } else {
-    hipLaunchKernelGGL((fmha_prefill_kernel<2, false>), dim3(tiles(64) * kHq), dim3(128),
-                       kFmLds, stream, qb, kb, vb, out, q_tokens, kv_tokens, tiles(64), none, ga);
+    hipLaunchKernelGGL((fmha_prefill_kernel<2, false>), grid(2), dim3(128), kFmLds, stream,
+                       qb, kb, vb, out, q_tokens, kv_tokens, tiles(2), none, ga);
   }
   return static_cast<int>(hipGetLastError());
 }
