@@ -611,6 +611,17 @@ size_t split_workspace_bytes(const SplitPlan& p) {
   return p.n_chunks > 1 ? (size_t)p.items * (p.waves * kFmRowsPerWave) * (kD + 2) * sizeof(float) : 0;
 }
 
+// Whether the call may run with this workspace, and whether it then splits.
+// Without enough of it, calls of up to 2560 tokens are refused and longer ones
+// run unsplit (they do not need the split to fill the GPU).
+bool split_workspace_ok(unsigned q_tokens, unsigned kv_tokens, const void* workspace,
+                        size_t workspace_bytes, bool* split) {
+  const size_t need = split_workspace_bytes(split_plan(q_tokens, kv_tokens));
+  const bool enough = workspace != nullptr && workspace_bytes >= need;
+  *split = need > 0 && enough;
+  return need == 0 || enough || q_tokens > 2560u;
+}
+
 bool valid_geometry(const void* q, const void* k, const void* v, const float* out,
                     unsigned q_tokens, unsigned kv_tokens) {
   return q != nullptr && k != nullptr && v != nullptr && out != nullptr && q_tokens != 0u &&
@@ -897,9 +908,10 @@ Q36_EXPORT int qwen36_fmha_prefill(const void* q, const void* k, const void* v, 
                                    unsigned query_tokens, unsigned kv_tokens, void* workspace,
                                    size_t workspace_bytes, void* stream) {
   if (!q36::valid_geometry(q, k, v, out, query_tokens, kv_tokens)) return Q36_EINVAL;
-  const size_t need = q36::split_workspace_bytes(q36::split_plan(query_tokens, kv_tokens));
-  if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return Q36_EINVAL;
-  return q36::launch_fmha(q, k, v, out, query_tokens, kv_tokens, need > 0 ? workspace : nullptr,
+  bool split = false;
+  if (!q36::split_workspace_ok(query_tokens, kv_tokens, workspace, workspace_bytes, &split))
+    return Q36_EINVAL;
+  return q36::launch_fmha(q, k, v, out, query_tokens, kv_tokens, split ? workspace : nullptr,
                           static_cast<hipStream_t>(stream));
 }
 
@@ -913,10 +925,11 @@ Q36_EXPORT int qwen36_fmha_prefill_gated(const void* q, const void* k, const voi
       (reinterpret_cast<uintptr_t>(q_gate) & 7u) != 0 || (q_gate_row_stride & 7u) != 0 ||
       (reinterpret_cast<uintptr_t>(out) & 15u) != 0)
     return Q36_EINVAL;
-  const size_t need = q36::split_workspace_bytes(q36::split_plan(query_tokens, kv_tokens));
-  if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return Q36_EINVAL;
+  bool split = false;
+  if (!q36::split_workspace_ok(query_tokens, kv_tokens, workspace, workspace_bytes, &split))
+    return Q36_EINVAL;
   const q36::GateArgs ga{static_cast<const q36::bf16*>(q_gate), q_gate_row_stride,
                          static_cast<q36::bf16*>(out)};
   return q36::launch_fmha(q, k, v, nullptr, query_tokens, kv_tokens,
-                          need > 0 ? workspace : nullptr, static_cast<hipStream_t>(stream), ga);
+                          split ? workspace : nullptr, static_cast<hipStream_t>(stream), ga);
 }

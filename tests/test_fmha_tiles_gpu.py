@@ -70,3 +70,21 @@ def test_provider_unsplit_tiles(gpu, t, s):
     ref = fmha_prefill(q, k, v)
     for out in outs:
         assert (out - ref).abs().max().item() <= 2 * TOL
+
+
+def test_long_split_without_workspace_runs_unsplit(gpu):
+    """2561 tokens and more split only if the caller gives the workspace; up
+    to 2560 a missing one is refused."""
+    from qwen36_attn import _lib
+    from qwen36_attn.full_attention import fmha_prefill
+    lib = _lib.load(("qwen36_fmha_prefill",))
+    t = 2561
+    assert lib.qwen36_fmha_prefill_workspace_bytes(t, t) > 0
+    g = torch.Generator().manual_seed(t)
+    q, k, v = (torch.randn(t, h, 256, generator=g).to(torch.bfloat16).to(gpu) for h in (16, 2, 2))
+    out = torch.empty(t, 4096, device=gpu)
+    st = torch.cuda.current_stream().cuda_stream
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr())
+    assert lib.qwen36_fmha_prefill(*args, 2560, 2560, None, 0, st) == 1
+    assert lib.qwen36_fmha_prefill(*args, t, t, None, 0, st) == 0
+    assert (out - fmha_prefill(q, k, v)).abs().max().item() <= 2 * TOL
