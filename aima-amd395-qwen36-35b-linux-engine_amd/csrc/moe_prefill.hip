@@ -18,8 +18,10 @@
 //   out = bf16(after + bf16(bf16(sum_k y_k) + shared))
 //
 // Launches (T tokens, E experts; the shared expert's rows are every token
-// in order, so its two GEMMs need no routing and run on a side stream,
-// forked after 1 and joined before 7, beside 2-4):
+// in order, so its two GEMMs need no routing and, from 2049 tokens on, run on
+// a side stream, forked after 1 and joined before 7, beside 2-4; shorter
+// prompts replace 5 and 6 by the streaming kernels of moe_stream.h, with the
+// shared expert as one more group):
 //  1. moe_pre_kernel       residual + RMSNorm, one wave per token.
 //  2. moe_gemm<kRouter>    logits [T, E + 1] = h2 [router | shared_gate]^T;
 //                          up to 8192 tokens in K slices whose fp32
@@ -27,9 +29,10 @@
 //  3. moe_topk_kernel      top-8 + routing softmax + shared gate, a wave per token.
 //  4. alignment            (token, rank) slots sorted by expert, each group
 //                          padded to 32 rows and cut into tiles of up to 128
-//                          rows: one workgroup up to 2048 tokens
-//                          (moe_align_one), else per-chunk histograms, one
-//                          scan workgroup and a per-chunk scatter.
+//                          rows (64 streaming), evenly: one workgroup up to
+//                          2048 tokens (moe_align_one), else per-chunk
+//                          histograms, one scan workgroup and a per-chunk
+//                          scatter.
 //  5. moe_gemm<kGateUp>    act [tile rows, 512] = silu(gate) * up per tile,
 //                          gate and up columns of one group in one workgroup
 //                          (side stream: the shared expert's T rows).
@@ -56,6 +59,7 @@
 // fetched byte for this tile; the tile shape was chosen from a sweep of
 // 64..256-row x 128..256-column tiles, K steps of 32/64 and 2..4 stages.
 #include "moe_common.h"
+#include "moe_stream.h"
 
 #include <algorithm>
 #include <mutex>
@@ -88,6 +92,13 @@ static_assert(kPfBK == 32 || kPfBK == 64, "K step");
 constexpr unsigned kPfMaxTokens = 262144;
 constexpr unsigned kAlignChunk = 4096;    // expert ids per histogram / scatter workgroup (least)
 constexpr unsigned kMaxAlignChunks = 256;
+// Up to this many tokens the expert GEMMs are the streaming kernels of
+// moe_stream.h (tiles of up to 64 rows) and the shared expert is one more
+// group of them: MI355X, whole block, against the 128-row kernel and a side
+// stream at every length: T = 5 69 us against 110, 45 226 / 263, 300 309 /
+// 350, 1000 343 / 411, 1400 372 / 452, 2048 462 / 477.  Longer prompts fill
+// 128-row tiles and take the kernel below (2100: 466 us).
+constexpr unsigned kStreamMaxTokens = 2048;
 
 enum GemmMode { kRouter = 0, kGateUp = 1, kDown = 2 };
 
@@ -107,12 +118,19 @@ struct PfLayout {
 // 4 slices slower there).
 unsigned router_splits(unsigned T) { return T <= 1024 ? 4u : T <= 8192 ? 2u : 1u; }
 
+// 128-column blocks per down workgroup of the streaming path: one while the
+// selected experts' items are few, then two to share the prologue (MI355X,
+// whole block: T = 2 49 us with 1, 52 with 2, 63 with 4; 45 236 / 239 / 248;
+// 128 285 / 281 / 308; 1000 343 / 342 / 354; 1400 380 / 373 / 381).
+unsigned stream_down_subs(unsigned T) { return T <= 64 ? 1u : 2u; }
+
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 PfLayout pf_layout(unsigned T, unsigned E) {
   PfLayout L;
   L.ld_logits = (E + 1 + 7) & ~7u;
-  L.max_tiles = (9u * T + kPfBM - 1) / kPfBM + E + 1;   // sum over groups of ceil(n / 128)
+  const unsigned bm = T <= kStreamMaxTokens ? kStBM : kPfBM;
+  L.max_tiles = (9u * T + bm - 1) / bm + E + 1;         // sum over groups of ceil(n / bm)
   L.max_rows = 9u * T + (kPfPad - 1) * (E + 1);         // sum of n rounded up to 32
   size_t o = 0;
   L.ids = o;     o = align256(o + (size_t)T * kMoeTopK * 4);
@@ -235,9 +253,12 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 
 // ---- 4. slots sorted by group, groups padded to 32 rows, 128-row tiles ----
 // sorted[p] = slot (t * 8 + k for routed rank k of token t) or -1 for
-// padding (the shared expert, every token, runs as launches of its own);
+// padding (the shared expert, every token, runs as launches of its own, or
+// is group E with slots 8T + t on the streaming path);
 // group g occupies rows [row_off[g], row_off[g] + roundup32(n_g)).  meta
-// (int4) [0] = {tiles}, [1 + i] = {group, first row, rows, 0} for tile i.
+// (int4) [0] = {tiles}, [1 + i] = {group, first row, rows, tiles of the
+// group} for tile i; a group's rows are dealt evenly to its tiles, so that
+// 130 rows make two tiles of 96 and 34 and not 128 and 2.
 // The 8T ids are cut into chunks of kAlignChunk: hist[g][chunk] counts, the
 // scan turns them into each chunk's first row per group, the scatter places
 // the chunk's slots.  Order inside a
@@ -280,6 +301,7 @@ __global__ __launch_bounds__(256) void moe_hist_kernel(const int* __restrict__ i
 // of the tiles (one wave's scans; [G] = totals), the tile table meta and
 // the padding rows of `sorted` (-1).  Called by every thread of the
 // workgroup; ends with the offsets visible to all of them.
+template <int kBM>
 __device__ __forceinline__ void group_offsets(const int* cnt, unsigned G, unsigned tid,
                                               int* row_off, int* tile_off,
                                               int4* __restrict__ meta,
@@ -292,7 +314,7 @@ __device__ __forceinline__ void group_offsets(const int* cnt, unsigned G, unsign
       const unsigned g = tid * kPer + j;
       const int c = g < G ? cnt[g] : 0;
       rows[j] = (c + kPfPad - 1) / kPfPad * kPfPad;
-      tiles[j] = (c + kPfBM - 1) / kPfBM;
+      tiles[j] = (c + kBM - 1) / kBM;
       rsum += rows[j];
       tsum += tiles[j];
     }
@@ -321,8 +343,10 @@ __device__ __forceinline__ void group_offsets(const int* cnt, unsigned G, unsign
   __syncthreads();
   for (unsigned g = tid; g < G; g += blockDim.x) {
     const int c = cnt[g], r0 = row_off[g];
-    for (int j = 0; j < tile_off[g + 1] - tile_off[g]; ++j)
-      meta[1 + tile_off[g] + j] = int4{(int)g, r0 + kPfBM * j, min(kPfBM, c - kPfBM * j), 0};
+    const int nt = tile_off[g + 1] - tile_off[g];
+    const int per = nt > 0 ? ((c + nt - 1) / nt + kPfPad - 1) / kPfPad * kPfPad : 0;
+    for (int j = 0; j < nt; ++j)
+      meta[1 + tile_off[g] + j] = int4{(int)g, r0 + per * j, max(0, min(per, c - per * j)), nt};
     for (int p = r0 + c; p < row_off[g + 1]; ++p) sorted[p] = -1;
   }
 }
@@ -350,7 +374,7 @@ __global__ __launch_bounds__(1024) void moe_scan_kernel(unsigned E, unsigned n_c
     if (tid == 0) cnt[E] = 0;   // the shared expert runs as launches of its own
   }
   __syncthreads();
-  group_offsets(cnt, G, tid, row_off, tile_off, meta, sorted);
+  group_offsets<kPfBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
   {   // chunk bases: one wave per group, exclusive prefix over the chunks
     const unsigned wave = tid >> 6, lane = tid & 63, waves = blockDim.x / 64;
     if (n_chunks <= 64) {   // every group's counts loaded up front (one round trip)
@@ -425,8 +449,11 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(const int* __restrict_
 
 // 4'. short prompts (8T <= kAlignOneIds): histogram, offsets and scatter in
 // one workgroup, the ids held in registers (16 per thread) -- one launch
-// instead of 4a-4c.
+// instead of 4a-4c.  kStream: tiles of 64 rows and the shared expert as group
+// E, every token in order.
 constexpr unsigned kAlignOneIds = 16384;
+static_assert(kMoeTopK * kStreamMaxTokens <= kAlignOneIds, "streaming aligns in one workgroup");
+template <bool kStream>
 __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restrict__ ids,
                                                              unsigned T, unsigned E,
                                                              int4* __restrict__ meta,
@@ -443,7 +470,7 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
     const unsigned i = tid + 1024 * u;
     v[u] = i < routed4 ? ids4[i] : int4{-1, -1, -1, -1};
   }
-  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = 0;   // [E]: shared expert, no rows
+  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = kStream && g == E ? (int)T : 0;
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
@@ -455,9 +482,11 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
     }
   }
   __syncthreads();
-  group_offsets(cnt, G, tid, row_off, tile_off, meta, sorted);
+  group_offsets<kStream ? kStBM : kPfBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
   __syncthreads();
   for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = row_off[g];   // next row per group
+  if constexpr (kStream)
+    for (unsigned t = tid; t < T; t += blockDim.x) sorted[row_off[E] + t] = (int)(kMoeTopK * T + t);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
@@ -541,7 +570,7 @@ __device__ __forceinline__ void gemm_k_loop(Fetch& fetch, const char* lds, int a
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb) {
           const bf16x8 a = *reinterpret_cast<const bf16x8*>(
-              st + (arow + 32 * rb) * kPfRowB + koff[s]);
+              st + (arow + 32 * (kPfBM / kPfWR) * rb) * kPfRowB + koff[s]);
           acc[rb][0] = mfma32x32x16(a, b0, acc[rb][0]);
           acc[rb][1] = mfma32x32x16(a, b1, acc[rb][1]);
         }
@@ -667,15 +696,16 @@ __global__ __launch_bounds__(64 * kPfWaves, kPfMinWG) void moe_gemm_kernel(GemmA
   };
 
   constexpr int kWm = kPfBM / kPfWR;
-  const int wm = wave % kWm, wn = wave / kWm;
+  constexpr int kWn = kPfWaves / kWm;
+  const int wm = wave / kWn, wn = wave % kWn;
   const int li = lane & 31, kh = lane >> 5;
-  const int arow = kPfWR * wm + li;
+  const int arow = 32 * wm + li;
   const int brow0 = kPfBM + (MODE == kGateUp ? 32 * wn + li : 64 * wn + li);
   const int brow1 = kPfBM + (MODE == kGateUp ? kPfBN / 2 + 32 * wn + li : 64 * wn + 32 + li);
   int koff[kPfBK / 16];
 #pragma unroll
   for (int s = 0; s < kPfBK / 16; ++s) koff[s] = (((2 * s + kh) ^ ((li / kPfRpw) % kPfCpr)) * 16);
-  const int nrb = min(kPfRB, max(0, (rows - kPfWR * wm + 31) / 32));
+  const int nrb = min(kPfRB, max(0, ((rows + 31) / 32 - wm + kWm - 1) / kWm));
 
   f32x16 acc[kPfRB][2];
 #pragma unroll
@@ -706,7 +736,7 @@ __global__ __launch_bounds__(64 * kPfWaves, kPfMinWG) void moe_gemm_kernel(GemmA
     if (rb >= nrb) break;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int r = kPfWR * wm + 32 * rb + 8 * (i >> 2) + 4 * kh + (i & 3);
+      const int r = 32 * (kWm * rb + wm) + 8 * (i >> 2) + 4 * kh + (i & 3);
       if (r >= rows) continue;
       if constexpr (MODE == kRouter && KS > 1) {
         const unsigned n = nt * kPfBN + 64 * wn + li;
@@ -835,6 +865,11 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
       const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kPfLds);
       if (e != hipSuccess) attr_status = e;
     }
+    for (const void* f : {reinterpret_cast<const void*>(moe_stream_kernel<false>),
+                          reinterpret_cast<const void*>(moe_stream_kernel<true>)}) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
+      if (e != hipSuccess) attr_status = e;
+    }
   });
   if (attr_status != hipSuccess) return (int)attr_status;
   const PfLayout L = pf_layout(T, E);
@@ -853,6 +888,53 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
   hipStream_t st = static_cast<hipStream_t>(stream);
   const unsigned tok_blocks = (T + 3) / 4;
 
+  hipLaunchKernelGGL(moe_pre_kernel, dim3(tok_blocks), dim3(256), 0, st,
+                     static_cast<const bf16*>(inp), static_cast<const bf16*>(attn_out),
+                     static_cast<const bf16*>(post_norm_w), after, h2, T);
+
+  GemmArgs g{};
+  g.T = T;
+  g.E = E;
+  g.meta = meta;
+  g.sorted = sorted;
+  g.rw = rw;
+  g.sgw = sgw;
+  auto grid_for = [](unsigned max_items) { return dim3(8 * ((max_items + 7) / 8)); };
+
+  const unsigned router_items = ((T + kPfBM - 1) / kPfBM) * n_blocks<kRouter>(E) * L.router_splits;
+  auto router = L.router_splits == 4   ? moe_gemm_kernel<kRouter, 4>
+                : L.router_splits == 2 ? moe_gemm_kernel<kRouter, 2>
+                                       : moe_gemm_kernel<kRouter>;
+  GemmArgs gr = g;
+  gr.a = h2;
+  gr.w = win;
+  gr.out = logits;
+  gr.ld_out = L.ld_logits;
+  gr.part = reinterpret_cast<float*>(ws + L.part);
+  gr.max_items = router_items;
+
+  if (T <= kStreamMaxTokens) {   // streaming path: one stream, the shared expert as group E
+    hipLaunchKernelGGL(router, grid_for(router_items), dim3(64 * kPfWaves), kPfLds, st, gr);
+    hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, gr.part,
+                       L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
+    hipLaunchKernelGGL(moe_align_one_kernel<true>, dim3(1), dim3(1024), 0, st, ids, T, E, meta,
+                       sorted);
+    StreamArgs a{h2, static_cast<const bf16*>(expert_gate_up), win + (size_t)(E + 1) * kMoeHidden,
+                 meta, sorted, rw, act, T, E, 1u};
+    hipLaunchKernelGGL(moe_stream_kernel<false>, grid_for(L.max_tiles * kStGateUpBlocks), dim3(512),
+                       kStLds, st, a);
+    a.a = act;
+    a.w = static_cast<const bf16*>(expert_down);
+    a.w_shared = static_cast<const bf16*>(shared_down);
+    a.out = y;
+    a.subs = stream_down_subs(T);
+    hipLaunchKernelGGL(moe_stream_kernel<true>, grid_for(L.max_tiles * (kStDownBlocks / a.subs)),
+                       dim3(512), kStLds, st, a);
+    hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, st, y, after, sgw,
+                       static_cast<bf16*>(out), T);
+    return static_cast<int>(hipGetLastError());
+  }
+
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPfMaxDevices) return Q36_EINVAL;
   std::lock_guard<std::mutex> lock(g_side_mutex);
@@ -868,18 +950,6 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
   }
   hipStream_t ss = side.s != nullptr ? side.s : st;
 
-  hipLaunchKernelGGL(moe_pre_kernel, dim3(tok_blocks), dim3(256), 0, st,
-                     static_cast<const bf16*>(inp), static_cast<const bf16*>(attn_out),
-                     static_cast<const bf16*>(post_norm_w), after, h2, T);
-
-  GemmArgs g{};
-  g.T = T;
-  g.E = E;
-  g.meta = meta;
-  g.sorted = sorted;
-  g.rw = rw;
-  g.sgw = sgw;
-  auto grid_for = [](unsigned max_items) { return dim3(8 * ((max_items + 7) / 8)); };
 
   // shared expert: gate/up then down (unscaled rows into its y slots) on
   // the side stream
@@ -905,31 +975,16 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
   hipLaunchKernelGGL(moe_gemm_kernel<kDown>, grid_for(gs.max_items), dim3(64 * kPfWaves), kPfLds, ss, gs);
   if (ss != st && hipEventRecord(side.join, ss) != hipSuccess) return static_cast<int>(hipGetLastError());
 
-  g.a = h2;
-  g.w = win;
-  g.out = logits;
-  g.ld_out = L.ld_logits;
-  g.part = reinterpret_cast<float*>(ws + L.part);
-  const unsigned router_items = ((T + kPfBM - 1) / kPfBM) * n_blocks<kRouter>(E) * L.router_splits;
-  g.max_items = router_items;
-  auto router = L.router_splits == 4   ? moe_gemm_kernel<kRouter, 4>
-                : L.router_splits == 2 ? moe_gemm_kernel<kRouter, 2>
-                                       : moe_gemm_kernel<kRouter>;
-  hipLaunchKernelGGL(router, grid_for(router_items), dim3(64 * kPfWaves), kPfLds, st, g);
-
-  hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, g.part,
+  hipLaunchKernelGGL(router, grid_for(router_items), dim3(64 * kPfWaves), kPfLds, st, gr);
+  hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, gr.part,
                      L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
-  if (kMoeTopK * T <= kAlignOneIds) {
-    hipLaunchKernelGGL(moe_align_one_kernel, dim3(1), dim3(1024), 0, st, ids, T, E, meta, sorted);
-  } else {
-    int* hist = reinterpret_cast<int*>(ws + L.hist);
-    hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
-                       L.n_chunks, L.chunk_ids, hist);
-    hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, st, E, L.n_chunks, hist, meta,
-                       sorted);
-    hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
-                       L.n_chunks, L.chunk_ids, hist, sorted);
-  }
+  int* hist = reinterpret_cast<int*>(ws + L.hist);
+  hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
+                     L.n_chunks, L.chunk_ids, hist);
+  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, st, E, L.n_chunks, hist, meta,
+                     sorted);
+  hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
+                     L.n_chunks, L.chunk_ids, hist, sorted);
 
   g.a = h2;
   g.w = static_cast<const bf16*>(expert_gate_up);
