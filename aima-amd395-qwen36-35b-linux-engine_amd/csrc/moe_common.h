@@ -14,6 +14,30 @@ constexpr float kMoeEps = 1e-6f;
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 
+// bf16(silu_f(g) * u) for a bf16 g, eight at a time: the SiLU from the
+// hardware exp2 and reciprocal (silu_fast's form, ~5 ulps from the exact one),
+// redone exactly where a product lies within 32 ulps of a bf16 rounding
+// midpoint (1 value in 1000), for |g| > 60 and for non-finite values, so the
+// bits are the exact form's at a third of its instructions.
+__device__ __forceinline__ void silu_mul8(const float (&g)[8], const float (&u)[8], bf16 (&o)[8]) {
+  float v[8];
+  bool slow = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float th = __builtin_amdgcn_exp2f(g[e] * -kLog2eHi);
+    const float t = __builtin_fmaf(th, g[e] * -kLn2Lo, th);
+    v[e] = (g[e] * __builtin_amdgcn_rcpf(1.0f + t)) * u[e];
+    const int mid = (int)(__float_as_uint(v[e]) & 0xffffu) - 0x8000;
+    slow |= !(fabsf(g[e]) <= 60.0f) || !(fabsf(v[e]) <= 3.0e38f) || (mid >= -32 && mid <= 32);
+  }
+  if (slow) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = silu_f(g[e]) * u[e];
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = f2bf(v[e]);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -17,49 +17,39 @@
 //           bf16(sigmoid(bf16(h2 . shared_gate)))
 //   out = bf16(after + bf16(bf16(sum_k y_k) + shared))
 //
-// Launches (T tokens, E experts; the shared expert's rows are every token
-// in order, so its two GEMMs need no routing and, from 2049 tokens on, run on
-// a side stream, forked after 1 and joined before 7, beside 2-4; shorter
-// prompts replace 5 and 6 by the streaming kernels of moe_stream.h, with the
-// shared expert as one more group):
+// Launches (T tokens, E experts; the shared expert is one more group of the
+// expert GEMMs, with every token):
 //  1. moe_pre_kernel       residual + RMSNorm, one wave per token.
-//  2. moe_gemm<kRouter>    logits [T, E + 1] = h2 [router | shared_gate]^T;
+//  2. moe_router_gemm      logits [T, E + 1] = h2 [router | shared_gate]^T;
 //                          up to 8192 tokens in K slices whose fp32
 //                          partials 3 sums.
 //  3. moe_topk_kernel      top-8 + routing softmax + shared gate, a wave per token.
 //  4. alignment            (token, rank) slots sorted by expert, each group
-//                          padded to 32 rows and cut into tiles of up to 128
-//                          rows (64 streaming), evenly: one workgroup up to
-//                          2048 tokens (moe_align_one), else per-chunk
+//                          padded to 32 rows and cut evenly into tiles of up
+//                          to 64 (short prompts) or 256 rows: one workgroup
+//                          up to 2048 tokens (moe_align_one), else per-chunk
 //                          histograms, one scan workgroup and a per-chunk
 //                          scatter.
-//  5. moe_gemm<kGateUp>    act [tile rows, 512] = silu(gate) * up per tile,
-//                          gate and up columns of one group in one workgroup
-//                          (side stream: the shared expert's T rows).
-//  6. moe_gemm<kDown>      y rows scaled by their routing weight, scattered to
-//                          their (token, rank) slot (side stream: the shared
-//                          rows, unscaled).
-//  7. moe_combine_kernel   per token: sum of the 8 routed rows, + the shared
-//                          row scaled by its gate, + after.
+//  5. gate/up              act [tile rows, 512] = silu(gate) * up per tile.
+//  6. down                 y rows, scattered to their (token, rank) slot
+//                          (5, 6: moe_stream.h up to 2048 tokens, moe_tile.h
+//                          above).
+//  7. moe_combine_kernel   per token: sum of the 8 weighted routed rows, + the
+//                          shared row scaled by its gate, + after.
 //
-// Grouped GEMM: a workgroup computes one tile of up to 128 rows of one
-// group against 256 weight rows, K in steps of 32, with 8 waves of 64 x 64 on
-// v_mfma_f32_32x32x16_bf16 (one 16-byte LDS read per MFMA); 32-row blocks past
-// the tile's rows are neither computed nor fetched.  Both operands are
-// K-contiguous in memory, so they are fetched straight into LDS
+// Router GEMM: a workgroup computes 128 tokens against 256 router rows, K in
+// steps of 32, with 8 waves of 64 x 64 on v_mfma_f32_32x32x16_bf16; 32-row
+// blocks past the last token are neither computed nor fetched.  Both operands
+// are K-contiguous in memory, so they are fetched straight into LDS
 // (buffer_load ... lds, 16 bytes per lane, 1 KiB per instruction) with an XOR
 // swizzle of the 16-byte chunks chosen by each lane's source address, which
 // makes the ds_read_b128 operand reads bank-conflict-free.  A 3-stage ring,
 // two workgroups per CU; the fetch is issued through inline asm (the
 // compiler would otherwise wait for it before reading the current stage) and
-// ordered by explicit vmcnt waits + barriers.  Work items (tile, column block)
-// are dealt to the 8 XCDs in contiguous ranges, so a tile's column blocks
-// and an expert's tiles share an L2.  Measured on MI355X: the loop is bound
-// by the L2/MALL -> LDS fill rate (~20-30 B/clk per CU), at ~87 flop per
-// fetched byte for this tile; the tile shape was chosen from a sweep of
-// 64..256-row x 128..256-column tiles, K steps of 32/64 and 2..4 stages.
+// ordered by explicit vmcnt waits + barriers.
 #include "moe_common.h"
 #include "moe_stream.h"
+#include "moe_tile.h"
 
 #include <algorithm>
 #include <mutex>
@@ -67,46 +57,39 @@
 namespace q36 {
 namespace {
 
-constexpr int kPfBM = 128;                // rows per tile (at most)
 constexpr int kPfPad = 32;                // group padding (rows)
-constexpr int kPfBN = 256;                // weight rows per workgroup
-constexpr int kPfWR = 64;                 // rows per wave (32-row blocks: kPfWR / 32)
-constexpr int kPfStages = 3;              // fetch ring depth
-constexpr int kPfMinWG = 2;               // workgroups per CU the kernel is built for
-constexpr int kPfBK = 32;                 // K per stage (32 or 64)
-constexpr int kPfRowB = kPfBK * 2;        // bytes per row per stage
-constexpr int kPfCpr = kPfRowB / 16;      // 16-byte chunks per row
-constexpr int kPfRpi = 1024 / kPfRowB;    // rows per fetch instruction
-constexpr int kPfRpw = 256 / kPfRowB;     // rows per 256-byte bank window
-constexpr int kPfAStage = kPfBM * kPfRowB;
-constexpr int kPfStage = kPfAStage + kPfBN * kPfRowB;
-constexpr int kPfLds = kPfStages * kPfStage;
-constexpr int kPfRB = kPfWR / 32;                        // row blocks per wave
-constexpr int kPfWaves = (kPfBM / kPfWR) * (kPfBN / 64); // each wave: kPfWR x 64
-constexpr int kPfInstr = (kPfBM + kPfBN) / kPfRpi / kPfWaves;  // fetch instructions per wave
-static_assert((kPfBM + kPfBN) / kPfRpi % kPfWaves == 0, "fetch split");
-static_assert(kPfBK == 32 || kPfBK == 64, "K step");
+// Router GEMM tile.
+constexpr int kRtBM = 128, kRtBN = 256;   // tokens, router rows per workgroup
+constexpr int kRtStages = 3;              // fetch ring depth
+constexpr int kRtBK = 32;                 // K per stage
+constexpr int kRtRowB = kRtBK * 2;        // bytes per row per stage
+constexpr int kRtCpr = kRtRowB / 16;      // 16-byte chunks per row
+constexpr int kRtRpi = 1024 / kRtRowB;    // rows per fetch instruction
+constexpr int kRtRpw = 256 / kRtRowB;     // rows per 256-byte bank window
+constexpr int kRtStage = (kRtBM + kRtBN) * kRtRowB;
+constexpr int kRtLds = kRtStages * kRtStage;
+constexpr int kRtWaves = 8;               // 2 x 4, each 64 tokens x 64 rows
+constexpr int kRtInstr = kRtStage / 1024 / kRtWaves;   // fetch instructions per wave
 // Swizzle: chunk c of stage row r sits at position c ^ key(r), key(r) =
-// (r / kPfRpw) % kPfCpr, so the 16 rows one ds_read_b128 pass serves fall in
+// (r / kRtRpw) % kRtCpr, so the 16 rows one ds_read_b128 pass serves fall in
 // 16 distinct 16-byte bank groups of the 256-byte bank window.
 constexpr unsigned kPfMaxTokens = 262144;
 constexpr unsigned kAlignChunk = 4096;    // expert ids per histogram / scatter workgroup (least)
 constexpr unsigned kMaxAlignChunks = 256;
 // Up to this many tokens the expert GEMMs are the streaming kernels of
 // moe_stream.h (tiles of up to 64 rows) and the shared expert is one more
-// group of them: MI355X, whole block, against the 128-row kernel and a side
-// stream at every length: T = 5 69 us against 110, 45 226 / 263, 300 309 /
-// 350, 1000 343 / 411, 1400 372 / 452, 2048 462 / 477.  Longer prompts fill
-// 128-row tiles and take the kernel below (2100: 466 us).
+// group of them: MI355X, whole block, against 128-row tiles and a side stream
+// at every length: T = 5 69 us against 110, 45 219 / 263, 300 309 / 350, 1000
+// 337 / 411, 1400 372 / 452, 2048 462 / 477.  Longer prompts take the 256-row
+// tiles of moe_tile.h (2100: 420 us against 476; one workgroup per CU and
+// whole weights per tile pay from about 128 rows a group).
 constexpr unsigned kStreamMaxTokens = 2048;
-
-enum GemmMode { kRouter = 0, kGateUp = 1, kDown = 2 };
 
 // Workspace layout for (T, E); every region 256-byte aligned.  The first
 // three regions (expert ids, routing weights, router logits) are read back by
 // the host's debug path at these fixed offsets.
 struct PfLayout {
-  size_t ids, rw, logits, sgw, meta, sorted, hist, after, h2, act, y, act_shared, part, total;
+  size_t ids, rw, logits, sgw, meta, sorted, hist, after, h2, act, y, part, total;
   unsigned ld_logits, max_tiles, max_rows, n_chunks, chunk_ids, router_splits;
 };
 
@@ -124,12 +107,16 @@ unsigned router_splits(unsigned T) { return T <= 1024 ? 4u : T <= 8192 ? 2u : 1u
 // 128 285 / 281 / 308; 1000 343 / 342 / 354; 1400 380 / 373 / 381).
 unsigned stream_down_subs(unsigned T) { return T <= 64 ? 1u : 2u; }
 
+// The same, 256 columns each, for the long-prompt down workgroups (whole
+// block: 4096 tokens 496 us with 1, 510 with 2; 8192 763 / 756).
+unsigned tile_down_subs(unsigned T) { return T <= 6144 ? 1u : 2u; }
+
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 PfLayout pf_layout(unsigned T, unsigned E) {
   PfLayout L;
   L.ld_logits = (E + 1 + 7) & ~7u;
-  const unsigned bm = T <= kStreamMaxTokens ? kStBM : kPfBM;
+  const unsigned bm = T <= kStreamMaxTokens ? kStBM : kTlBM;
   L.max_tiles = (9u * T + bm - 1) / bm + E + 1;         // sum over groups of ceil(n / bm)
   L.max_rows = 9u * T + (kPfPad - 1) * (E + 1);         // sum of n rounded up to 32
   size_t o = 0;
@@ -147,7 +134,6 @@ PfLayout pf_layout(unsigned T, unsigned E) {
   L.h2 = o;      o = align256(o + (size_t)T * kMoeHidden * 2);
   L.act = o;     o = align256(o + (size_t)L.max_rows * kMoeInter * 2);
   L.y = o;       o = align256(o + (size_t)9 * T * kMoeHidden * 2);
-  L.act_shared = o;  o = align256(o + (size_t)T * kMoeInter * 2);
   L.router_splits = router_splits(T);
   L.part = o;
   if (L.router_splits > 1) o = align256(o + (size_t)L.router_splits * T * L.ld_logits * 4);
@@ -251,10 +237,9 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
   if (lane == 0) sgw[t] = bf2f(f2bf(1.0f / (1.0f + expf(-sg_logit))));
 }
 
-// ---- 4. slots sorted by group, groups padded to 32 rows, 128-row tiles ----
+// ---- 4. slots sorted by group, groups padded to 32 rows, tiles ------------
 // sorted[p] = slot (t * 8 + k for routed rank k of token t) or -1 for
-// padding (the shared expert, every token, runs as launches of its own, or
-// is group E with slots 8T + t on the streaming path);
+// padding; the shared expert is group E with slots 8T + t;
 // group g occupies rows [row_off[g], row_off[g] + roundup32(n_g)).  meta
 // (int4) [0] = {tiles}, [1 + i] = {group, first row, rows, tiles of the
 // group} for tile i; a group's rows are dealt evenly to its tiles, so that
@@ -354,7 +339,7 @@ __device__ __forceinline__ void group_offsets(const int* cnt, unsigned G, unsign
 // 4b. one workgroup: group totals, row / tile offsets (one-wave scans), tile
 // table, padding, shared-expert rows, and hist turned into each chunk's
 // first row per group.
-__global__ __launch_bounds__(1024) void moe_scan_kernel(unsigned E, unsigned n_chunks,
+__global__ __launch_bounds__(1024) void moe_scan_kernel(unsigned T, unsigned E, unsigned n_chunks,
                                                         int* __restrict__ hist,
                                                         int4* __restrict__ meta,
                                                         int* __restrict__ sorted) {
@@ -371,10 +356,11 @@ __global__ __launch_bounds__(1024) void moe_scan_kernel(unsigned E, unsigned n_c
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
     if (g < E && part == 0) cnt[g] = sum;
-    if (tid == 0) cnt[E] = 0;   // the shared expert runs as launches of its own
+    if (tid == 0) cnt[E] = (int)T;   // the shared expert: every token
   }
   __syncthreads();
-  group_offsets<kPfBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
+  group_offsets<kTlBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
+  for (unsigned t = tid; t < T; t += blockDim.x) sorted[row_off[E] + t] = (int)(kMoeTopK * T + t);
   {   // chunk bases: one wave per group, exclusive prefix over the chunks
     const unsigned wave = tid >> 6, lane = tid & 63, waves = blockDim.x / 64;
     if (n_chunks <= 64) {   // every group's counts loaded up front (one round trip)
@@ -449,11 +435,9 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(const int* __restrict_
 
 // 4'. short prompts (8T <= kAlignOneIds): histogram, offsets and scatter in
 // one workgroup, the ids held in registers (16 per thread) -- one launch
-// instead of 4a-4c.  kStream: tiles of 64 rows and the shared expert as group
-// E, every token in order.
+// instead of 4a-4c, with tiles of 64 rows.
 constexpr unsigned kAlignOneIds = 16384;
 static_assert(kMoeTopK * kStreamMaxTokens <= kAlignOneIds, "streaming aligns in one workgroup");
-template <bool kStream>
 __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restrict__ ids,
                                                              unsigned T, unsigned E,
                                                              int4* __restrict__ meta,
@@ -470,7 +454,7 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
     const unsigned i = tid + 1024 * u;
     v[u] = i < routed4 ? ids4[i] : int4{-1, -1, -1, -1};
   }
-  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = kStream && g == E ? (int)T : 0;
+  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = g == E ? (int)T : 0;
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
@@ -482,11 +466,10 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
     }
   }
   __syncthreads();
-  group_offsets<kStream ? kStBM : kPfBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
+  group_offsets<kStBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
   __syncthreads();
   for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = row_off[g];   // next row per group
-  if constexpr (kStream)
-    for (unsigned t = tid; t < T; t += blockDim.x) sorted[row_off[E] + t] = (int)(kMoeTopK * T + t);
+  for (unsigned t = tid; t < T; t += blockDim.x) sorted[row_off[E] + t] = (int)(kMoeTopK * T + t);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
@@ -500,77 +483,43 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
   }
 }
 
-// ---- 2/5/6. grouped GEMM ----------------------------------------------------
-struct GemmArgs {
-  const bf16* a;            // h2 [T, 2048] (router, gate/up) or act [rows, 512] (down)
-  const bf16* w;            // router: w_in; gate/up: expert_gate_up; down: expert_down
-  const bf16* w_shared;     // gate/up: shared [gate_proj | up_proj]; down: shared_down
-  const int4* meta;
-  const int* sorted;
-  const float* rw;
-  const float* sgw;
-  bf16* out;                // logits / act / y
-  float* part;              // router with K slices: fp32 partials [slices][T][ld_out]
-  unsigned T, E, ld_out, max_items;
-  unsigned shared;          // gate/up, down: the shared expert's T rows in token order
+// ---- 2. router GEMM -----------------------------------------------------------
+struct RouterArgs {
+  const bf16* a;            // h2 [T, 2048]
+  const bf16* w;            // w_in: router and shared-gate rows first
+  bf16* out;                // logits [T, ld]
+  float* part;              // K slices: fp32 partials [slices][T][ld]
+  unsigned T, E, ld;
 };
 
-// The leading s_nop covers a hazard the compiler cannot see through the
-// inline assembly: the resource SGPRs (and m0) are written by VALU
-// readfirstlane / SALU instructions right before, and a VMEM instruction
-// reading an SGPR that a VALU wrote needs 5 wait states on gfx950 (issued
-// earlier, it reads the old descriptor).
-__device__ __forceinline__ void fetch_rows(unsigned lds_addr, int voff, const u32x4& rsrc) {
-  asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-               :: "v"(voff), "s"(rsrc), "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr))
-               : "memory");
-}
+unsigned router_blocks(unsigned E) { return (E + kRtBN) / kRtBN; }   // of its E + 1 rows
 
-__device__ __forceinline__ u32x4 buffer_rsrc(const void* base, unsigned bytes) {
-  const unsigned long long a = reinterpret_cast<unsigned long long>(base);
-  return u32x4{(unsigned)a, (unsigned)(a >> 32), bytes, 0x00020000u};
-}
-
-constexpr unsigned kOob = 0x80000000u;   // a row offset past every buffer's range
-
-template <int MODE>
-__host__ __device__ constexpr unsigned n_blocks(unsigned E) {
-  return MODE == kRouter ? (E + 1 + kPfBN - 1) / kPfBN
-                         : (MODE == kGateUp ? kMoeInter / (kPfBN / 2) : kMoeHidden / kPfBN);
-}
-
-// s_waitcnt immediate that waits until at most n vector-memory operations of
-// this wave are outstanding (expcnt and lgkmcnt not waited on).
-constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// The K loop for a wave computing NRB (0..kPfRB) row blocks of 32.  Every
-// wave fetches and meets the barriers whatever its NRB.  Stage s of the ring
-// holds K step s mod kPfStages; the fetch of step + kPfStages - 1 is issued
+// The K loop for a wave computing NRB (0..2) row blocks of 32.  Every wave
+// fetches and meets the barriers whatever its NRB.  Stage s of the ring
+// holds K step s mod kRtStages; the fetch of step + kRtStages - 1 is issued
 // once every wave has finished reading step - 1.
 template <int NRB, int NSTEPS, typename Fetch>
-__device__ __forceinline__ void gemm_k_loop(Fetch& fetch, const char* lds, int arow, int brow0,
-                                            int brow1, const int (&koff)[kPfBK / 16],
-                                            f32x16 (&acc)[kPfRB][2]) {
+__device__ __forceinline__ void router_k_loop(Fetch& fetch, const char* lds, int arow, int brow,
+                                              const int (&koff)[kRtBK / 16], f32x16 (&acc)[2][2]) {
 #pragma unroll
-  for (int st = 0; st < kPfStages - 1; ++st) fetch(st);
+  for (int st = 0; st < kRtStages - 1; ++st) fetch(st);
   for (int step = 0; step < NSTEPS; ++step) {
     // this wave's fetches of `step` landed (later ones may stay in flight)
-    if (step + kPfStages - 2 < NSTEPS)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm((kPfStages - 2) * kPfInstr));
+    if (step + kRtStages - 2 < NSTEPS)
+      __builtin_amdgcn_s_waitcnt(stream_vmcnt((kRtStages - 2) * kRtInstr));
     else
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      __builtin_amdgcn_s_waitcnt(stream_vmcnt(0));
     __syncthreads();   // every wave's fetches landed; stage (step - 1) is free
-    if (step + kPfStages - 1 < NSTEPS) fetch(step + kPfStages - 1);
+    if (step + kRtStages - 1 < NSTEPS) fetch(step + kRtStages - 1);
     if constexpr (NRB > 0) {
-      const char* st = lds + (step % kPfStages) * kPfStage;
+      const char* st = lds + (step % kRtStages) * kRtStage;
 #pragma unroll
-      for (int s = 0; s < kPfBK / 16; ++s) {
-        const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(st + brow0 * kPfRowB + koff[s]);
-        const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(st + brow1 * kPfRowB + koff[s]);
+      for (int s = 0; s < kRtBK / 16; ++s) {
+        const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(st + brow * kRtRowB + koff[s]);
+        const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(st + (brow + 32) * kRtRowB + koff[s]);
 #pragma unroll
         for (int rb = 0; rb < NRB; ++rb) {
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>(
-              st + (arow + 32 * (kPfBM / kPfWR) * rb) * kPfRowB + koff[s]);
+          const bf16x8 a = *reinterpret_cast<const bf16x8*>(st + (arow + 32 * rb) * kRtRowB + koff[s]);
           acc[rb][0] = mfma32x32x16(a, b0, acc[rb][0]);
           acc[rb][1] = mfma32x32x16(a, b1, acc[rb][1]);
         }
@@ -579,23 +528,18 @@ __device__ __forceinline__ void gemm_k_loop(Fetch& fetch, const char* lds, int a
   }
 }
 
-// Wave (wm = w % (BM / WR), wn = w / (BM / WR)) computes tile rows
-// WR wm + 32 rb against weight rows (gate/up: gate 32wn.. and up BN/2 +
-// 32wn.., i.e. act columns 32wn..; else 64wn.. and 64wn + 32..).  Fetch
-// instruction i (of (BM + BN) / 8) moves rows 8i..8i+7 of the stage: A rows
-// first, then B rows; wave w issues instructions w * kPfInstr + j.
-// KS > 1 (router only): item i covers K slice i % KS of tile i / KS.
-template <int MODE, int KS = 1>
-__global__ __launch_bounds__(64 * kPfWaves, kPfMinWG) void moe_gemm_kernel(GemmArgs p) {
-  static_assert(KS == 1 || MODE == kRouter, "K slices are for the router");
+// Wave (wm = w % 2, wn = w / 2) computes tokens 64 wm .. + 63 against rows
+// 64 wn .. + 63.  Fetch instruction i moves rows 16i .. 16i + 15 of the stage,
+// token rows first; wave w issues instructions kRtInstr w + j.  Workgroup i
+// covers K slice i % KS of tile i / KS, tiles dealt to the XCDs in
+// contiguous ranges.
+template <int KS>
+__global__ __launch_bounds__(64 * kRtWaves, 2) void moe_router_gemm_kernel(RouterArgs p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  constexpr int K = MODE == kDown ? kMoeInter : kMoeHidden;
-  constexpr int nsteps = K / kPfBK / KS;
-  static_assert(nsteps * kPfBK * KS == K, "K slices");
-  const unsigned nb = n_blocks<MODE>(p.E);
-  const unsigned m_tiles = (MODE == kRouter || p.shared) ? (p.T + kPfBM - 1) / kPfBM
-                                                          : (unsigned)p.meta[0].x;
-  const unsigned items = m_tiles * nb * KS;
+  constexpr int nsteps = kMoeHidden / kRtBK / KS;
+  static_assert(nsteps * kRtBK * KS == kMoeHidden, "K slices");
+  const unsigned nb = (p.E + kRtBN) / kRtBN;
+  const unsigned items = (p.T + kRtBM - 1) / kRtBM * nb * KS;
   const unsigned share = (items + 7) / 8;
   const unsigned xi = blockIdx.x >> 3;
   if (xi >= share) return;
@@ -603,78 +547,22 @@ __global__ __launch_bounds__(64 * kPfWaves, kPfMinWG) void moe_gemm_kernel(GemmA
   if (item >= items) return;
   const unsigned ks = item % KS;
   const unsigned mt = item / KS / nb, nt = item / KS % nb;
-  int group = 0, row0, rows;
-  if (MODE == kRouter || p.shared) {
-    group = MODE == kRouter ? 0 : (int)p.E;
-    row0 = (int)(mt * kPfBM);
-    rows = min(kPfBM, (int)p.T - row0);
-  } else {
-    const int4 m = p.meta[1 + mt];
-    group = m.x;
-    row0 = m.y;
-    rows = m.z;
-  }
+  const int row0 = (int)(mt * kRtBM), rows = min(kRtBM, (int)p.T - row0);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-
   // Operand sources (buffer resources: out-of-range rows read as zero).
-  u32x4 ars, brs;
-  if constexpr (MODE == kDown)
-    ars = buffer_rsrc(p.a + (size_t)row0 * kMoeInter, (unsigned)rows * kMoeInter * 2u);
-  else
-    ars = buffer_rsrc(p.a, p.T * (unsigned)kMoeHidden * 2u);
-  if constexpr (MODE == kRouter) {
-    brs = buffer_rsrc(p.w, (p.E + 1) * (unsigned)kMoeHidden * 2u);
-  } else if constexpr (MODE == kGateUp) {
-    const bf16* wg = group < (int)p.E ? p.w + (size_t)group * (2 * kMoeInter) * kMoeHidden
-                                      : p.w_shared;
-    brs = buffer_rsrc(wg, 2u * kMoeInter * kMoeHidden * 2u);
-  } else {
-    const bf16* wg = group < (int)p.E ? p.w + (size_t)group * kMoeHidden * kMoeInter
-                                      : p.w_shared;
-    brs = buffer_rsrc(wg, (unsigned)kMoeHidden * kMoeInter * 2u);
-  }
-
-  // Fetch plan: one instruction moves 1 KiB, kPfRpi rows of kPfRowB bytes
-  // (lane = row in the instruction x chunk position; the source chunk is
-  // position ^ key(row), so LDS holds the swizzled layout).  A instructions
-  // whose rows are all past the tile's rows load nothing (an out-of-range
-  // offset), which keeps every wave's count of loads per stage equal.
-  const int rin = lane / kPfCpr, cpos = lane % kPfCpr;   // row in the instruction, chunk
-  unsigned f_off[kPfInstr];
-  u32x4 f_rs[kPfInstr];
-  bool f_live[kPfInstr];
+  const u32x4 ars = stream_rsrc(p.a, p.T * (unsigned)kMoeHidden * 2u);
+  const u32x4 brs = stream_rsrc(p.w, (p.E + 1) * (unsigned)kMoeHidden * 2u);
+  const int rin = lane / kRtCpr, cpos = lane % kRtCpr;   // row in the instruction, chunk
+  unsigned f_off[kRtInstr];
+  u32x4 f_rs[kRtInstr];
 #pragma unroll
-  for (int j = 0; j < kPfInstr; ++j) {
-    const int ins = wave * kPfInstr + j;
-    const bool is_a = ins < kPfBM / kPfRpi;
-    unsigned off;
-    if (is_a) {
-      const int r = ins * kPfRpi + rin;
-      if constexpr (MODE == kRouter) {
-        off = r < rows ? (unsigned)(row0 + r) * kMoeHidden * 2u : kOob;
-      } else if constexpr (MODE == kGateUp) {
-        const int slot = r >= rows ? -1
-                         : p.shared ? (int)(kMoeTopK * p.T) + row0 + r : p.sorted[row0 + r];
-        const unsigned routed = kMoeTopK * p.T;
-        const unsigned t = slot < 0 ? 0u : ((unsigned)slot < routed ? (unsigned)slot / kMoeTopK
-                                                                    : (unsigned)slot - routed);
-        off = slot < 0 ? kOob : t * (unsigned)kMoeHidden * 2u;
-      } else {
-        off = (unsigned)r * kMoeInter * 2u;
-      }
-    } else {
-      const int r = (ins - kPfBM / kPfRpi) * kPfRpi + rin;
-      unsigned row;
-      if constexpr (MODE == kGateUp)
-        row = r < kPfBN / 2 ? nt * (kPfBN / 2) + r : kMoeInter + nt * (kPfBN / 2) + (r - kPfBN / 2);
-      else
-        row = nt * kPfBN + r;
-      off = row * (unsigned)K * 2u;
-    }
-    const int srow = ins * kPfRpi + rin;   // stage row this lane fills
-    f_off[j] = off + ((cpos ^ ((srow / kPfRpw) % kPfCpr)) * 16);
-    f_live[j] = !is_a || ins * kPfRpi < rows;
+  for (int j = 0; j < kRtInstr; ++j) {
+    const int srow = (wave * kRtInstr + j) * kRtRpi + rin;   // stage row this lane fills
+    const bool is_a = srow < kRtBM;   // (uniform: an instruction's rows are of one operand)
+    const unsigned off = !is_a ? (nt * kRtBN + srow - kRtBM) * (unsigned)kMoeHidden * 2u
+                         : srow < rows ? (unsigned)(row0 + srow) * kMoeHidden * 2u : kStOob;
+    f_off[j] = off + ((cpos ^ ((srow / kRtRpw) % kRtCpr)) * 16);
     const u32x4 r = is_a ? ars : brs;
 #pragma unroll
     for (int c = 0; c < 4; ++c) f_rs[j][c] = __builtin_amdgcn_readfirstlane(r[c]);
@@ -682,99 +570,59 @@ __global__ __launch_bounds__(64 * kPfWaves, kPfMinWG) void moe_gemm_kernel(GemmA
   const unsigned lds0 = static_cast<unsigned>(
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
   auto fetch = [&](int step) {
-    const unsigned sbase = lds0 + (step % kPfStages) * kPfStage;
-    const unsigned kb = (ks * nsteps + (unsigned)step) * kPfRowB;
+    const unsigned sbase = lds0 + (step % kRtStages) * kRtStage;
+    const unsigned kb = (ks * nsteps + (unsigned)step) * kRtRowB;
 #pragma unroll
-    for (int j = 0; j < kPfInstr; ++j) {
-      // a dead instruction is still issued, with an out-of-range offset (no
-      // memory is read), so every wave keeps the same count of outstanding
-      // loads per stage for the vmcnt waits
-      const int ins = wave * kPfInstr + j;
-      fetch_rows(sbase + ins * kPfRpi * kPfRowB, f_live[j] ? (int)(f_off[j] + kb) : (int)kOob,
-                 f_rs[j]);
-    }
+    for (int j = 0; j < kRtInstr; ++j)
+      stream_fetch<false>(sbase + (wave * kRtInstr + j) * 1024, (int)(f_off[j] + kb), f_rs[j]);
   };
 
-  constexpr int kWm = kPfBM / kPfWR;
-  constexpr int kWn = kPfWaves / kWm;
-  const int wm = wave / kWn, wn = wave % kWn;
+  const int wm = wave % 2, wn = wave / 2;
   const int li = lane & 31, kh = lane >> 5;
-  const int arow = 32 * wm + li;
-  const int brow0 = kPfBM + (MODE == kGateUp ? 32 * wn + li : 64 * wn + li);
-  const int brow1 = kPfBM + (MODE == kGateUp ? kPfBN / 2 + 32 * wn + li : 64 * wn + 32 + li);
-  int koff[kPfBK / 16];
+  const int arow = 64 * wm + li, brow = kRtBM + 64 * wn + li;
+  int koff[kRtBK / 16];
 #pragma unroll
-  for (int s = 0; s < kPfBK / 16; ++s) koff[s] = (((2 * s + kh) ^ ((li / kPfRpw) % kPfCpr)) * 16);
-  const int nrb = min(kPfRB, max(0, ((rows + 31) / 32 - wm + kWm - 1) / kWm));
+  for (int s = 0; s < kRtBK / 16; ++s) koff[s] = (((2 * s + kh) ^ ((li / kRtRpw) % kRtCpr)) * 16);
+  const int nrb = min(2, max(0, (rows - 64 * wm + 31) / 32));
 
-  f32x16 acc[kPfRB][2];
+  f32x16 acc[2][2];
 #pragma unroll
-  for (int i = 0; i < kPfRB; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  if (nrb == 0) {
-    gemm_k_loop<0, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc);
-  } else if constexpr (kPfRB == 1) {
-    gemm_k_loop<1, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc);
-  } else if constexpr (kPfRB == 2) {
-    if (nrb == 1) gemm_k_loop<1, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc);
-    else gemm_k_loop<2, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc);
-  } else {
-    switch (nrb) {
-      case 1: gemm_k_loop<1, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc); break;
-      case 2: gemm_k_loop<2, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc); break;
-      case 3: gemm_k_loop<3, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc); break;
-      default: gemm_k_loop<kPfRB, nsteps>(fetch, lds, arow, brow0, brow1, koff, acc); break;
-    }
-  }
+  for (int i = 0; i < 2; ++i) acc[i][0] = acc[i][1] = f32x16{};
+  if (nrb == 2) router_k_loop<2, nsteps>(fetch, lds, arow, brow, koff, acc);
+  else if (nrb == 1) router_k_loop<1, nsteps>(fetch, lds, arow, brow, koff, acc);
+  else router_k_loop<0, nsteps>(fetch, lds, arow, brow, koff, acc);
 
-  // acc[rb][cb][i] = tile row WR wm + 32rb + 8(i/4) + 4kh + i%4, weight row
-  // brow_cb.
-  const unsigned routed = kMoeTopK * p.T;
+  // acc[rb][cb][i] = token 64 wm + 32 rb + 8(i/4) + 4kh + i%4, router row n + 32 cb
+  const unsigned n = nt * kRtBN + 64 * wn + li;
 #pragma unroll
-  for (int rb = 0; rb < kPfRB; ++rb) {
+  for (int rb = 0; rb < 2; ++rb) {
     if (rb >= nrb) break;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int r = 32 * (kWm * rb + wm) + 8 * (i >> 2) + 4 * kh + (i & 3);
+      const int r = 64 * wm + 32 * rb + 8 * (i >> 2) + 4 * kh + (i & 3);
       if (r >= rows) continue;
-      if constexpr (MODE == kRouter && KS > 1) {
-        const unsigned n = nt * kPfBN + 64 * wn + li;
-        float* o = p.part + ((size_t)ks * p.T + row0 + r) * p.ld_out;
+      if constexpr (KS > 1) {
+        float* o = p.part + ((size_t)ks * p.T + row0 + r) * p.ld;
         if (n <= p.E) o[n] = acc[rb][0][i];
         if (n + 32 <= p.E) o[n + 32] = acc[rb][1][i];
-      } else if constexpr (MODE == kRouter) {
-        const unsigned n = nt * kPfBN + 64 * wn + li;
-        bf16* o = p.out + (size_t)(row0 + r) * p.ld_out;
+      } else {
+        bf16* o = p.out + (size_t)(row0 + r) * p.ld;
         if (n <= p.E) o[n] = f2bf(acc[rb][0][i]);
         if (n + 32 <= p.E) o[n + 32] = f2bf(acc[rb][1][i]);
-      } else if constexpr (MODE == kGateUp) {
-        const unsigned c = nt * (kPfBN / 2) + 32 * wn + li;
-        const float g = bf2f(f2bf(acc[rb][0][i])), u = bf2f(f2bf(acc[rb][1][i]));
-        p.out[(size_t)(row0 + r) * kMoeInter + c] = f2bf(silu_f(g) * u);
-      } else if (p.shared) {
-        // the shared expert's row, unscaled: the combine applies the shared
-        // gate (known only after the router) with this epilogue's roundings
-        bf16* y = p.out + (size_t)(routed + row0 + r) * kMoeHidden + nt * kPfBN + 64 * wn + li;
-        y[0] = f2bf(acc[rb][0][i]);
-        y[32] = f2bf(acc[rb][1][i]);
-      } else {
-        const int slot = p.sorted[row0 + r];
-        const float w = p.rw[slot];
-        bf16* y = p.out + (size_t)slot * kMoeHidden + nt * kPfBN + 64 * wn + li;
-        y[0] = f2bf(bf2f(f2bf(acc[rb][0][i])) * w);
-        y[32] = f2bf(bf2f(f2bf(acc[rb][1][i])) * w);
       }
     }
   }
 }
 
 // ---- 7. per-token combine --------------------------------------------------
+// kWeigh: the rows arrive unscaled (streaming path) and are scaled here, with
+// the down epilogue's roundings.
 // moe = bf16(sum over ranks 0..7 of y, fp32 in rank order); out = bf16(after +
 // bf16(moe + shared)) -- the order of qwen36_moe_decode's combine.
+template <bool kWeigh>
 __global__ __launch_bounds__(256) void moe_combine_kernel(
-    const bf16* __restrict__ y, const bf16* __restrict__ after, const float* __restrict__ sgw,
-    bf16* __restrict__ out, unsigned T) {
+    const bf16* __restrict__ y, const float* __restrict__ rw, const bf16* __restrict__ after,
+    const float* __restrict__ sgw, bf16* __restrict__ out, unsigned T) {
   const unsigned t = blockIdx.x;
   const int c = 8 * threadIdx.x;
   float moe[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -789,7 +637,10 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 #pragma unroll
   for (int k = 0; k < kMoeTopK; ++k)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) moe[e] += bf2f(yk[k][e]);
+    for (int e = 0; e < 8; ++e) {
+      const float v = bf2f(yk[k][e]);
+      moe[e] += kWeigh ? bf2f(f2bf(v * rw[(size_t)t * kMoeTopK + k])) : v;
+    }
   bf16x8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -799,23 +650,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   }
   *reinterpret_cast<bf16x8*>(out + (size_t)t * kMoeHidden + c) = o;
 }
-
-// The shared expert depends only on the normalised rows (its gate is applied
-// in the combine), so its two GEMMs run on a side stream while the router,
-// top-8 and alignment chain -- a few latency-bound launches that leave most
-// CUs idle -- runs on the caller's stream, and the routed GEMMs then hold
-// only the routed tiles.  One side stream and a fork / join event pair per
-// device, created on first use; the mutex keeps each call's record / wait
-// pairs together when several host threads enqueue at once.  If they cannot
-// be created, everything runs on the caller's stream.
-constexpr int kPfMaxDevices = 64;
-struct SideStream {
-  bool tried = false;
-  hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-std::mutex g_side_mutex;
-SideStream g_side[kPfMaxDevices];
 
 }  // namespace
 }  // namespace q36
@@ -854,22 +688,20 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
       !aligned16(workspace))
     return Q36_EINVAL;
   const unsigned T = tokens, E = n_experts;
-  static std::once_flag attr_once;   // 80 KiB of dynamic LDS per GEMM workgroup
+  static std::once_flag attr_once;   // 72 to 160 KiB of dynamic LDS per GEMM workgroup
   static hipError_t attr_status = hipSuccess;
   std::call_once(attr_once, [] {
-    for (const void* f : {reinterpret_cast<const void*>(moe_gemm_kernel<kRouter>),
-                          reinterpret_cast<const void*>(moe_gemm_kernel<kRouter, 2>),
-                          reinterpret_cast<const void*>(moe_gemm_kernel<kRouter, 4>),
-                          reinterpret_cast<const void*>(moe_gemm_kernel<kGateUp>),
-                          reinterpret_cast<const void*>(moe_gemm_kernel<kDown>)}) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kPfLds);
+    auto allow = [](const void* f, int bytes) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
       if (e != hipSuccess) attr_status = e;
-    }
-    for (const void* f : {reinterpret_cast<const void*>(moe_stream_kernel<false>),
-                          reinterpret_cast<const void*>(moe_stream_kernel<true>)}) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
-      if (e != hipSuccess) attr_status = e;
-    }
+    };
+    allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<1>), kRtLds);
+    allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<2>), kRtLds);
+    allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<4>), kRtLds);
+    allow(reinterpret_cast<const void*>(moe_stream_kernel<false>), kStLds);
+    allow(reinterpret_cast<const void*>(moe_stream_kernel<true>), kStLds);
+    allow(reinterpret_cast<const void*>(moe_tile_kernel<false>), kTlLds);
+    allow(reinterpret_cast<const void*>(moe_tile_kernel<true>), kTlLds);
   });
   if (attr_status != hipSuccess) return (int)attr_status;
   const PfLayout L = pf_layout(T, E);
@@ -892,117 +724,44 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
                      static_cast<const bf16*>(inp), static_cast<const bf16*>(attn_out),
                      static_cast<const bf16*>(post_norm_w), after, h2, T);
 
-  GemmArgs g{};
-  g.T = T;
-  g.E = E;
-  g.meta = meta;
-  g.sorted = sorted;
-  g.rw = rw;
-  g.sgw = sgw;
   auto grid_for = [](unsigned max_items) { return dim3(8 * ((max_items + 7) / 8)); };
+  const RouterArgs r{h2, win, logits, reinterpret_cast<float*>(ws + L.part), T, E, L.ld_logits};
+  auto router = L.router_splits == 4   ? moe_router_gemm_kernel<4>
+                : L.router_splits == 2 ? moe_router_gemm_kernel<2>
+                                       : moe_router_gemm_kernel<1>;
+  hipLaunchKernelGGL(router, grid_for((T + kRtBM - 1) / kRtBM * router_blocks(E) * L.router_splits),
+                     dim3(64 * kRtWaves), kRtLds, st, r);
+  hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, r.part,
+                     L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
 
-  const unsigned router_items = ((T + kPfBM - 1) / kPfBM) * n_blocks<kRouter>(E) * L.router_splits;
-  auto router = L.router_splits == 4   ? moe_gemm_kernel<kRouter, 4>
-                : L.router_splits == 2 ? moe_gemm_kernel<kRouter, 2>
-                                       : moe_gemm_kernel<kRouter>;
-  GemmArgs gr = g;
-  gr.a = h2;
-  gr.w = win;
-  gr.out = logits;
-  gr.ld_out = L.ld_logits;
-  gr.part = reinterpret_cast<float*>(ws + L.part);
-  gr.max_items = router_items;
-
-  if (T <= kStreamMaxTokens) {   // streaming path: one stream, the shared expert as group E
-    hipLaunchKernelGGL(router, grid_for(router_items), dim3(64 * kPfWaves), kPfLds, st, gr);
-    hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, gr.part,
-                       L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
-    hipLaunchKernelGGL(moe_align_one_kernel<true>, dim3(1), dim3(1024), 0, st, ids, T, E, meta,
-                       sorted);
-    StreamArgs a{h2, static_cast<const bf16*>(expert_gate_up), win + (size_t)(E + 1) * kMoeHidden,
-                 meta, sorted, rw, act, T, E, 1u};
+  StreamArgs a{h2, static_cast<const bf16*>(expert_gate_up), win + (size_t)(E + 1) * kMoeHidden,
+               meta, sorted, rw, act, T, E, 1u};
+  StreamArgs d{act, static_cast<const bf16*>(expert_down), static_cast<const bf16*>(shared_down),
+               meta, sorted, rw, y, T, E, 1u};
+  if (T <= kStreamMaxTokens) {
+    hipLaunchKernelGGL(moe_align_one_kernel, dim3(1), dim3(1024), 0, st, ids, T, E, meta, sorted);
     hipLaunchKernelGGL(moe_stream_kernel<false>, grid_for(L.max_tiles * kStGateUpBlocks), dim3(512),
                        kStLds, st, a);
-    a.a = act;
-    a.w = static_cast<const bf16*>(expert_down);
-    a.w_shared = static_cast<const bf16*>(shared_down);
-    a.out = y;
-    a.subs = stream_down_subs(T);
-    hipLaunchKernelGGL(moe_stream_kernel<true>, grid_for(L.max_tiles * (kStDownBlocks / a.subs)),
-                       dim3(512), kStLds, st, a);
-    hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, st, y, after, sgw,
+    d.subs = stream_down_subs(T);
+    hipLaunchKernelGGL(moe_stream_kernel<true>, grid_for(L.max_tiles * (kStDownBlocks / d.subs)),
+                       dim3(512), kStLds, st, d);
+    hipLaunchKernelGGL(moe_combine_kernel<true>, dim3(T), dim3(256), 0, st, y, rw, after, sgw,
                        static_cast<bf16*>(out), T);
-    return static_cast<int>(hipGetLastError());
+  } else {
+    int* hist = reinterpret_cast<int*>(ws + L.hist);
+    hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
+                       L.n_chunks, L.chunk_ids, hist);
+    hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, st, T, E, L.n_chunks, hist, meta,
+                       sorted);
+    hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
+                       L.n_chunks, L.chunk_ids, hist, sorted);
+    hipLaunchKernelGGL(moe_tile_kernel<false>, grid_for(L.max_tiles * kTlGateUpBlocks),
+                       dim3(64 * kTlWaves), kTlLds, st, a);
+    d.subs = tile_down_subs(T);
+    hipLaunchKernelGGL(moe_tile_kernel<true>, grid_for(L.max_tiles * (kTlDownBlocks / d.subs)),
+                       dim3(64 * kTlWaves), kTlLds, st, d);
+    hipLaunchKernelGGL(moe_combine_kernel<false>, dim3(T), dim3(256), 0, st, y, rw, after, sgw,
+                       static_cast<bf16*>(out), T);
   }
-
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPfMaxDevices) return Q36_EINVAL;
-  std::lock_guard<std::mutex> lock(g_side_mutex);
-  SideStream& side = g_side[dev];
-  if (!side.tried) {
-    side.tried = true;
-    if (hipStreamCreateWithFlags(&side.s, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&side.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&side.join, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      side.s = nullptr;
-    }
-  }
-  hipStream_t ss = side.s != nullptr ? side.s : st;
-
-
-  // shared expert: gate/up then down (unscaled rows into its y slots) on
-  // the side stream
-  if (ss != st) {
-    if (hipEventRecord(side.fork, st) != hipSuccess || hipStreamWaitEvent(ss, side.fork, 0) != hipSuccess)
-      return static_cast<int>(hipGetLastError());
-  }
-  bf16* act_shared = reinterpret_cast<bf16*>(ws + L.act_shared);
-  const unsigned shared_items = (T + kPfBM - 1) / kPfBM;
-  GemmArgs gs = g;
-  gs.shared = 1;
-  gs.a = h2;
-  gs.w = static_cast<const bf16*>(expert_gate_up);
-  gs.w_shared = win + (size_t)(E + 1) * kMoeHidden;
-  gs.out = act_shared;
-  gs.max_items = shared_items * n_blocks<kGateUp>(E);
-  hipLaunchKernelGGL(moe_gemm_kernel<kGateUp>, grid_for(gs.max_items), dim3(64 * kPfWaves), kPfLds, ss, gs);
-  gs.a = act_shared;
-  gs.w = static_cast<const bf16*>(expert_down);
-  gs.w_shared = static_cast<const bf16*>(shared_down);
-  gs.out = y;
-  gs.max_items = shared_items * n_blocks<kDown>(E);
-  hipLaunchKernelGGL(moe_gemm_kernel<kDown>, grid_for(gs.max_items), dim3(64 * kPfWaves), kPfLds, ss, gs);
-  if (ss != st && hipEventRecord(side.join, ss) != hipSuccess) return static_cast<int>(hipGetLastError());
-
-  hipLaunchKernelGGL(router, grid_for(router_items), dim3(64 * kPfWaves), kPfLds, st, gr);
-  hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, gr.part,
-                     L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
-  int* hist = reinterpret_cast<int*>(ws + L.hist);
-  hipLaunchKernelGGL(moe_hist_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
-                     L.n_chunks, L.chunk_ids, hist);
-  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, st, E, L.n_chunks, hist, meta,
-                     sorted);
-  hipLaunchKernelGGL(moe_scatter_kernel, dim3(L.n_chunks), dim3(256), 0, st, ids, T, E,
-                     L.n_chunks, L.chunk_ids, hist, sorted);
-
-  g.a = h2;
-  g.w = static_cast<const bf16*>(expert_gate_up);
-  g.w_shared = win + (size_t)(E + 1) * kMoeHidden;
-  g.out = act;
-  g.max_items = L.max_tiles * n_blocks<kGateUp>(E);
-  hipLaunchKernelGGL(moe_gemm_kernel<kGateUp>, grid_for(g.max_items), dim3(64 * kPfWaves), kPfLds, st, g);
-
-  g.a = act;
-  g.w = static_cast<const bf16*>(expert_down);
-  g.w_shared = static_cast<const bf16*>(shared_down);
-  g.out = y;
-  g.max_items = L.max_tiles * n_blocks<kDown>(E);
-  hipLaunchKernelGGL(moe_gemm_kernel<kDown>, grid_for(g.max_items), dim3(64 * kPfWaves), kPfLds, st, g);
-
-  if (ss != st && hipStreamWaitEvent(st, side.join, 0) != hipSuccess)
-    return static_cast<int>(hipGetLastError());
-  hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, st, y, after, sgw,
-                     static_cast<bf16*>(out), T);
   return static_cast<int>(hipGetLastError());
 }

@@ -24,6 +24,8 @@
 namespace q36 {
 namespace {
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
 constexpr int kStBM = 64;                  // rows per tile (at most)
 constexpr int kStBN = 128;                 // weight rows per block
 constexpr int kStRowB = 128;               // bytes per row and step (64 K)
@@ -40,13 +42,24 @@ struct StreamArgs {
   const bf16* w_shared;   // group E: the shared expert's
   const int4* meta;       // [0].x tiles; [1 + i] = {group, first row, rows, tiles of the group}
   const int* sorted;      // slot of each row: t * 8 + k, or 8 T + t (shared)
-  const float* rw;        // routing weight of each routed slot
+  const float* rw;        // routing weight of each routed slot (long prompts' down)
   bf16* out;              // act [rows, 512] / y [9 T, 2048]
   unsigned T, E, subs;    // subs (down): 128-column blocks per workgroup
 };
 
-// One 1 KiB fetch, as fetch_rows of the long-prompt GEMM (the s_nop covers
-// the VALU-written resource SGPRs), with or without the nontemporal hint.
+// Buffer resource over `bytes` bytes: reads past them give zeros.
+__device__ __forceinline__ u32x4 stream_rsrc(const void* base, unsigned bytes) {
+  const unsigned long long a = reinterpret_cast<unsigned long long>(base);
+  return u32x4{(unsigned)a, (unsigned)(a >> 32), bytes, 0x00020000u};
+}
+constexpr unsigned kStOob = 0x80000000u;   // an offset past every buffer's range
+
+// One 1 KiB fetch into LDS, with or without the nontemporal hint.  The
+// leading s_nop covers a hazard the compiler cannot see through the
+// inline assembly: the resource SGPRs (and m0) are written by VALU
+// readfirstlane / SALU instructions right before, and a VMEM instruction
+// reading an SGPR that a VALU wrote needs 5 wait states on gfx950 (issued
+// earlier, it reads the old descriptor).
 template <bool kNt>
 __device__ __forceinline__ void stream_fetch(unsigned lds_addr, int voff, const u32x4& rsrc) {
   if constexpr (kNt)
@@ -57,6 +70,11 @@ __device__ __forceinline__ void stream_fetch(unsigned lds_addr, int voff, const 
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                  :: "v"(voff), "s"(rsrc), "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr))
                  : "memory");
+}
+
+// v of the lane beside (lane ^ 1), by DPP.
+__device__ __forceinline__ float beside(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
 }
 
 // s_waitcnt immediate: at most n vector-memory operations outstanding.
@@ -93,16 +111,12 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
   u32x4 ars, brs, yrs;
   const bf16* wg = group < (int)p.E ? p.w + (size_t)group * (kDown ? 1 : 2) * kMoeInter * kMoeHidden
                                     : p.w_shared;
-  auto rsrc_of = [](const void* base, unsigned bytes) {
-    const unsigned long long a = reinterpret_cast<unsigned long long>(base);
-    return u32x4{(unsigned)a, (unsigned)(a >> 32), bytes, 0x00020000u};
-  };
-  brs = rsrc_of(wg, (kDown ? 1u : 2u) * kMoeInter * kMoeHidden * 2u);
-  yrs = rsrc_of(p.out, kDown ? 9u * p.T * (unsigned)kMoeHidden * 2u : 0u);
+  brs = stream_rsrc(wg, (kDown ? 1u : 2u) * kMoeInter * kMoeHidden * 2u);
+  yrs = stream_rsrc(p.out, kDown ? 9u * p.T * (unsigned)kMoeHidden * 2u : 0u);
   if constexpr (kDown)
-    ars = rsrc_of(p.a + (size_t)row0 * kMoeInter, (unsigned)rows * kMoeInter * 2u);
+    ars = stream_rsrc(p.a + (size_t)row0 * kMoeInter, (unsigned)rows * kMoeInter * 2u);
   else
-    ars = rsrc_of(p.a, p.T * (unsigned)kMoeHidden * 2u);
+    ars = stream_rsrc(p.a, p.T * (unsigned)kMoeHidden * 2u);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     ars[c] = __builtin_amdgcn_readfirstlane(ars[c]);
@@ -114,7 +128,6 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
   // first), lane = row in the instruction x chunk position; a wave issues
   // instructions kStIns * wave + j.  Rows past the tile's end are fetched
   // out of range (nothing is read).
-  constexpr unsigned kOobRow = 0x80000000u;
   const int rin = lane >> 3, cpos = lane & 7;
   unsigned f_off[kStIns];
 #pragma unroll
@@ -123,11 +136,11 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
     unsigned off;
     if (srow < kStBM) {
       if constexpr (kDown) {
-        off = srow < rows ? (unsigned)srow * kMoeInter * 2u : kOobRow;
+        off = srow < rows ? (unsigned)srow * kMoeInter * 2u : kStOob;
       } else {
         const int slot = srow < rows ? p.sorted[row0 + srow] : -1;
         const unsigned t = (unsigned)slot < routed ? (unsigned)slot / kMoeTopK : (unsigned)slot - routed;
-        off = slot < 0 ? kOobRow : t * (unsigned)kMoeHidden * 2u;
+        off = slot < 0 ? kStOob : t * (unsigned)kMoeHidden * 2u;
       }
     } else {
       const int r = srow - kStBM;
@@ -181,15 +194,13 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
   // lane's j-th.  Rows past the tile's end are stored out of range.
   constexpr int kStores = kDown ? 8 : 0;
   unsigned y_off[kDown ? 8 : 1];
-  float y_w[kDown ? 8 : 1];
   if constexpr (kDown) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int i = 2 * j + (li & 1);
       const int r = 32 * wm + 8 * (i >> 2) + 4 * kh + (i & 3);
       const int slot = r < rows ? p.sorted[row0 + r] : -1;
-      y_off[j] = slot < 0 ? kOobRow : (unsigned)slot * (kMoeHidden * 2u);
-      y_w[j] = slot >= 0 && (unsigned)slot < routed ? p.rw[slot] : 1.0f;
+      y_off[j] = slot < 0 ? kStOob : (unsigned)slot * (kMoeHidden * 2u);
     }
   }
 
@@ -227,10 +238,8 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float keep = odd ? acc[2 * j + 1] : acc[2 * j];
-          const float got = __shfl_xor(odd ? acc[2 * j] : acc[2 * j + 1], 1, 64);
-          const float lo = bf2f(f2bf(odd ? got : keep)), hi = bf2f(f2bf(odd ? keep : got));
-          typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-          const bf16x2 v = {f2bf(lo * y_w[j]), f2bf(hi * y_w[j])};
+          const float got = beside(odd ? acc[2 * j] : acc[2 * j + 1]);
+          const bf16x2 v = {f2bf(odd ? got : keep), f2bf(odd ? keep : got)};
           stream_store(__builtin_bit_cast(unsigned, v), (int)(y_off[j] + 2 * c), yrs);
         }
         acc = f32x16{};
@@ -243,14 +252,20 @@ __global__ __launch_bounds__(512, 4) void moe_stream_kernel(StreamArgs p) {
     // the low lanes finish rows of acc[0..7], the high lanes acc[8..15]
     const bool hi = (li & 16) != 0;
     const unsigned c = nt * (kStBN / 2) + 16 * wn + (li & 15);
+    float g8[8], u8[8];
+    bf16 a8[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float other = __shfl_xor(hi ? acc[i] : acc[i + 8], 16, 64);
-      const float g = hi ? other : acc[i], u = hi ? acc[i + 8] : other;
+      g8[i] = bf2f(f2bf(hi ? other : acc[i]));
+      u8[i] = bf2f(f2bf(hi ? acc[i + 8] : other));
+    }
+    silu_mul8(g8, u8, a8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
       const int q = hi ? i + 8 : i;
       const int r = 32 * wm + 8 * (q >> 2) + 4 * kh + (q & 3);
-      if (r < rows)
-        p.out[(size_t)(row0 + r) * kMoeInter + c] = f2bf(silu_f(bf2f(f2bf(g))) * bf2f(f2bf(u)));
+      if (r < rows) p.out[(size_t)(row0 + r) * kMoeInter + c] = a8[i];
     }
   }
 }
