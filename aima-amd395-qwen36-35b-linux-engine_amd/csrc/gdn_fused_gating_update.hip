@@ -13,12 +13,20 @@
 //
 // In this orientation every state row evolves on its own: the two
 // reductions of a token (H k, H q) run along a row, so a row is owned by 8
-// lanes (16 key columns each) and reduced by three shuffles, with no LDS and
+// lanes (16 key columns each, as four pieces 32 columns apart, so that one
+// load of the 8 lanes covers a 128-byte line) and reduced by three shuffles, with no LDS and
 // no barrier.  The squared norms of q and k and q.k come out of the same
 // shuffles (the 8 lanes of a row cover all 128 key columns), and
 // o = e^g (H_old q) + v' (k.q) (H' q expanded) keeps one reduction round per
 // token.  grid = 32 heads x 8 blocks of 16 rows; 128 threads; the state is
 // read once and written once per call (state_out may alias state_in).
+//
+// HBM-bound from about 8 sequences: 4.2 MB of state each, read and written.
+// MI355X, us per call over pools larger than the Infinity Cache (16 columns
+// side by side per lane, 64-byte strides / this layout / and nontemporal): 1
+// sequence 4.2 / 3.7 / 3.5, 8 13.1 / 9.9 / 7.2, 48 50 / 41 / 37, 256 226 / 206 /
+// 184 (5.8 TB/s).  Two rows per lane group (fewer q, k loads) 38 at 48, 197
+// at 256.
 #include "common.h"
 
 namespace q36 {
@@ -26,7 +34,7 @@ namespace {
 
 constexpr int kFguRows = 16;                    // state rows per workgroup
 constexpr int kFguLanesPerRow = 8;
-constexpr int kFguCols = kGdnDk / kFguLanesPerRow;   // 16 key columns per lane
+static_assert(kGdnDk == 16 * kFguLanesPerRow, "16 key columns per lane");
 
 __global__ __launch_bounds__(kFguRows * kFguLanesPerRow) void gdn_fused_gating_update_kernel(
     const float* __restrict__ a_log, const bf16* __restrict__ a,
@@ -57,41 +65,42 @@ __global__ __launch_bounds__(kFguRows * kFguLanesPerRow) void gdn_fused_gating_u
   state_out += slot;
   const int row = blockIdx.y * kFguRows + (threadIdx.x / kFguLanesPerRow);
   const int part = threadIdx.x % kFguLanesPerRow;
-  const int c0 = part * kFguCols;
   const int kh = h * (int)qk_heads / kGdnHv;
-  float* so = state_out + ((size_t)h * kGdnDv + row) * kGdnDk + c0;
-  const float* si = state_in + ((size_t)h * kGdnDv + row) * kGdnDk + c0;
-  float s[kFguCols];
+  // lane `part` of a row owns columns 4 part + 32 j .. + 3, j < 4
+  const size_t at = ((size_t)h * kGdnDv + row) * kGdnDk + 4 * part;
+  f32x4 s[4];
 #pragma unroll
-  for (int i = 0; i < kFguCols; i += 4) {
-    const f32x4 x = *reinterpret_cast<const f32x4*>(si + i);
-    s[i] = x[0]; s[i + 1] = x[1]; s[i + 2] = x[2]; s[i + 3] = x[3];
-  }
+  for (int j = 0; j < 4; ++j)
+    s[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state_in + at + 32 * j));
   const float A = expf(a_log[h]);
   const float dtb = dt_bias[h];
   for (unsigned t = t_begin; t < t_end; ++t) {
     // every per-token input is requested up front (one memory round trip)
-    const bf16x8* qp = reinterpret_cast<const bf16x8*>(q + (size_t)t * qk_token_stride + kh * kGdnDk + c0);
-    const bf16x8* kp = reinterpret_cast<const bf16x8*>(k + (size_t)t * qk_token_stride + kh * kGdnDk + c0);
-    const bf16x8 q0 = qp[0], q1 = qp[1], k0 = kp[0], k1 = kp[1];
+    const bf16* qp = q + (size_t)t * qk_token_stride + kh * kGdnDk + 4 * part;
+    const bf16* kp = k + (size_t)t * qk_token_stride + kh * kGdnDk + 4 * part;
+    bf16x4 qr[4], kr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      qr[j] = *reinterpret_cast<const bf16x4*>(qp + 32 * j);
+      kr[j] = *reinterpret_cast<const bf16x4*>(kp + 32 * j);
+    }
     const float vv = bf2f(v[(size_t)t * v_token_stride + h * kGdnDv + row]);
     const float av = bf2f(a[(size_t)t * ab_row_stride + h]);
     const float bv = bf2f(b[(size_t)t * ab_row_stride + h]);
-    float qf[kFguCols], kf[kFguCols];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      qf[i] = bf2f(q0[i]); qf[8 + i] = bf2f(q1[i]);
-      kf[i] = bf2f(k0[i]); kf[8 + i] = bf2f(k1[i]);
-    }
+    f32x4 kf[4];
     float hk = 0.f, hq = 0.f, kk = 0.f, qq = 0.f, kq = 0.f;
 #pragma unroll
-    for (int i = 0; i < kFguCols; ++i) {
-      hk += s[i] * kf[i];
-      hq += s[i] * qf[i];
-      kk += kf[i] * kf[i];
-      qq += qf[i] * qf[i];
-      kq += kf[i] * qf[i];
-    }
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float qv = bf2f(qr[j][i]), kv = bf2f(kr[j][i]);
+        kf[j][i] = kv;
+        hk += s[j][i] * kv;
+        hq += s[j][i] * qv;
+        kk += kv * kv;
+        qq += qv * qv;
+        kq += kv * qv;
+      }
 #pragma unroll
     for (int o = 1; o < kFguLanesPerRow; o <<= 1) {
       hk += __shfl_xor(hk, o, 64);
@@ -110,12 +119,14 @@ __global__ __launch_bounds__(kFguRows * kFguLanesPerRow) void gdn_fused_gating_u
     const float o = eg * (hq * qn) + vn * ((kq * kinv) * qn);
     const float vk = vn * kinv;
 #pragma unroll
-    for (int i = 0; i < kFguCols; ++i) s[i] = s[i] * eg + vk * kf[i];
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[j][i] = s[j][i] * eg + vk * kf[j][i];
     if (part == 0) out[((size_t)t * kGdnHv + h) * kGdnDv + row] = f2bf(o);
   }
 #pragma unroll
-  for (int i = 0; i < kFguCols; i += 4)
-    *reinterpret_cast<f32x4*>(so + i) = f32x4{s[i], s[i + 1], s[i + 2], s[i + 3]};
+  for (int j = 0; j < 4; ++j)
+    __builtin_nontemporal_store(s[j], reinterpret_cast<f32x4*>(state_out + at + 32 * j));
 }
 
 }  // namespace
