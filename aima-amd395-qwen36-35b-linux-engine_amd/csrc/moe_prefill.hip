@@ -178,16 +178,15 @@ __global__ __launch_bounds__(256) void moe_pre_kernel(
 }
 
 // ---- 3. top-8 + routing weights + shared gate, one wave per token ---------
-// With `splits` > 1 the router GEMM left fp32 partials of its K slices
-// (part [splits][T][ld]): the wave sums them in slice order, rounds to bf16
-// and writes the logits row itself.
-__global__ __launch_bounds__(256) void moe_topk_kernel(
-    bf16* __restrict__ logits, const float* __restrict__ part, unsigned splits, unsigned ld,
-    unsigned E, unsigned T, int* __restrict__ ids_out, float* __restrict__ rw_out,
+// Token t's part by one wave; lane k < 8 returns the id of rank k.  With
+// `splits` > 1 the router GEMM left fp32 partials of its K slices (part
+// [splits][T][ld]): the wave sums them in slice order, rounds to bf16 and
+// writes the logits row itself.
+__device__ __forceinline__ int topk_token(
+    unsigned t, bf16* __restrict__ logits, const float* __restrict__ part, unsigned splits,
+    unsigned ld, unsigned E, unsigned T, int* __restrict__ ids_out, float* __restrict__ rw_out,
     float* __restrict__ sgw) {
   const int lane = threadIdx.x & 63;
-  const unsigned t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;
   bf16* row = logits + (size_t)t * ld;
   int ids[kMoeTopK];
   float vals[kMoeTopK], rw[kMoeTopK];
@@ -223,18 +222,27 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
     sg_logit = bf2f(row[E]);
   }
   routing_weights(vals, rw);
-  if (lane < kMoeTopK) {
-    int id = ids[0];
-    float w = rw[0];
+  int id = ids[0];
+  float w = rw[0];
 #pragma unroll
-    for (int k = 1; k < kMoeTopK; ++k) {
-      id = lane == k ? ids[k] : id;
-      w = lane == k ? rw[k] : w;
-    }
+  for (int k = 1; k < kMoeTopK; ++k) {
+    id = lane == k ? ids[k] : id;
+    w = lane == k ? rw[k] : w;
+  }
+  if (lane < kMoeTopK) {
     ids_out[(size_t)t * kMoeTopK + lane] = id;
     rw_out[(size_t)t * kMoeTopK + lane] = w;
   }
   if (lane == 0) sgw[t] = bf2f(f2bf(1.0f / (1.0f + expf(-sg_logit))));
+  return id;
+}
+
+__global__ __launch_bounds__(256) void moe_topk_kernel(
+    bf16* __restrict__ logits, const float* __restrict__ part, unsigned splits, unsigned ld,
+    unsigned E, unsigned T, int* __restrict__ ids_out, float* __restrict__ rw_out,
+    float* __restrict__ sgw) {
+  const unsigned t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t < T) topk_token(t, logits, part, splits, ld, E, T, ids_out, rw_out, sgw);
 }
 
 // ---- 4. slots sorted by group, groups padded to 32 rows, tiles ------------
@@ -483,6 +491,39 @@ __global__ __launch_bounds__(1024) void moe_align_one_kernel(const int* __restri
   }
 }
 
+// 3 + 4 in one workgroup for up to kFewTokens tokens, a wave each: the ids go
+// to the alignment through LDS (whole block, 2 .. 8 tokens: 1.4 us less; more
+// tokens per wave cost more than the launch they save: 64 tokens 260 us
+// against 249).
+constexpr unsigned kFewTokens = 16;
+__global__ __launch_bounds__(1024) void moe_topk_align_few_kernel(
+    bf16* __restrict__ logits, const float* __restrict__ part, unsigned splits, unsigned ld,
+    unsigned E, unsigned T, int* __restrict__ ids_out, float* __restrict__ rw_out,
+    float* __restrict__ sgw, int4* __restrict__ meta, int* __restrict__ sorted) {
+  __shared__ int cnt[kMoeMaxExperts + 1];
+  __shared__ int row_off[kMoeMaxExperts + 2];
+  __shared__ int tile_off[kMoeMaxExperts + 2];
+  __shared__ int ids[kFewTokens * kMoeTopK];
+  const unsigned G = E + 1, tid = threadIdx.x;
+  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = g == E ? (int)T : 0;
+  __syncthreads();
+  const unsigned t = tid >> 6;
+  if (t < T) {
+    const int id = topk_token(t, logits, part, splits, ld, E, T, ids_out, rw_out, sgw);
+    if ((tid & 63) < (unsigned)kMoeTopK) {
+      ids[t * kMoeTopK + (tid & 63)] = id;
+      atomicAdd(&cnt[id], 1);
+    }
+  }
+  __syncthreads();
+  group_offsets<kStBM>(cnt, G, tid, row_off, tile_off, meta, sorted);
+  __syncthreads();
+  for (unsigned g = tid; g < G; g += blockDim.x) cnt[g] = row_off[g];   // next row per group
+  if (tid < T) sorted[row_off[E] + tid] = (int)(kMoeTopK * T + tid);
+  __syncthreads();
+  if (tid < kMoeTopK * T) sorted[atomicAdd(&cnt[ids[tid]], 1)] = (int)tid;
+}
+
 // ---- 2. router GEMM -----------------------------------------------------------
 struct RouterArgs {
   const bf16* a;            // h2 [T, 2048]
@@ -614,6 +655,60 @@ __global__ __launch_bounds__(64 * kRtWaves, 2) void moe_router_gemm_kernel(Route
   }
 }
 
+// The same in four K slices for short prompts: a workgroup takes 64 tokens,
+// 32 router rows and one slice of 512 K, fetches all of it at once (96 KiB,
+// one row per instruction) and multiplies it from LDS -- one round trip where
+// the ring above makes one per 32 K.  Chunk c of row r sits at c ^ (r % 16).
+// The products and their order are those of the ring's slices.  MI355X, whole
+// block, against the ring: 2 tokens 46.6 us / 48.1, 45 225 / 229, 300 296 /
+// 302, 600 317 / 318; from there on the ring's larger tiles win (1000: 339 /
+// 335).
+constexpr unsigned kRsMaxTokens = 512;
+constexpr int kRsTokens = 64, kRsRows = 32, kRsRowB = kMoeHidden / 4 * 2;
+constexpr int kRsLds = (kRsTokens + kRsRows) * kRsRowB;
+__global__ __launch_bounds__(256) void moe_router_short_kernel(RouterArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const unsigned n0 = blockIdx.x * kRsRows, ks = blockIdx.y, row0 = blockIdx.z * kRsTokens;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  u32x4 ars = stream_rsrc(p.a, p.T * (unsigned)kMoeHidden * 2u);
+  u32x4 brs = stream_rsrc(p.w, (p.E + 1) * (unsigned)kMoeHidden * 2u);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    ars[c] = __builtin_amdgcn_readfirstlane(ars[c]);
+    brs[c] = __builtin_amdgcn_readfirstlane(brs[c]);
+  }
+  const unsigned lds0 = static_cast<unsigned>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
+  const int rows = min(kRsTokens, (int)(p.T - row0));
+  // rows past the last token or router row read as zeros
+  for (int r = wave; r < kRsTokens + kRsRows; r += 4) {
+    const unsigned off = ks * kRsRowB + ((lane ^ (r & 15)) * 16);
+    if (r >= kRsTokens)
+      stream_fetch<false>(lds0 + r * kRsRowB, (int)((n0 + r - kRsTokens) * kMoeHidden * 2u + off), brs);
+    else if (r < (rows + 31) / 32 * 32)
+      stream_fetch<false>(lds0 + r * kRsRowB, (int)((row0 + r) * kMoeHidden * 2u + off), ars);
+  }
+  __builtin_amdgcn_s_waitcnt(stream_vmcnt(0));
+  __syncthreads();
+  if (32 * wave >= rows) return;   // waves 0 and 1 own 32 tokens each
+  const int li = lane & 31, kh = lane >> 5;
+  const char* ap = lds + (32 * wave + li) * kRsRowB;
+  const char* bp = lds + (kRsTokens + li) * kRsRowB;
+  f32x16 acc = f32x16{};
+#pragma unroll 8
+  for (int s = 0; s < kRsRowB / 32; ++s) {
+    const int at = ((2 * s + kh) ^ (li & 15)) * 16;
+    acc = mfma32x32x16(*reinterpret_cast<const bf16x8*>(ap + at),
+                       *reinterpret_cast<const bf16x8*>(bp + at), acc);
+  }
+  const unsigned n = n0 + li;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = 32 * wave + 8 * (i >> 2) + 4 * kh + (i & 3);
+    if (r < rows && n <= p.E) p.part[((size_t)ks * p.T + row0 + r) * p.ld + n] = acc[i];
+  }
+}
+
 // ---- 7. per-token combine --------------------------------------------------
 // kWeigh: the rows arrive unscaled (streaming path) and are scaled here, with
 // the down epilogue's roundings.
@@ -698,6 +793,7 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
     allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<1>), kRtLds);
     allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<2>), kRtLds);
     allow(reinterpret_cast<const void*>(moe_router_gemm_kernel<4>), kRtLds);
+    allow(reinterpret_cast<const void*>(moe_router_short_kernel), kRsLds);
     allow(reinterpret_cast<const void*>(moe_stream_kernel<false>), kStLds);
     allow(reinterpret_cast<const void*>(moe_stream_kernel<true>), kStLds);
     allow(reinterpret_cast<const void*>(moe_tile_kernel<false>), kTlLds);
@@ -726,20 +822,31 @@ Q36_EXPORT int qwen36_moe_prefill(const void* inp, const void* attn_out, const v
 
   auto grid_for = [](unsigned max_items) { return dim3(8 * ((max_items + 7) / 8)); };
   const RouterArgs r{h2, win, logits, reinterpret_cast<float*>(ws + L.part), T, E, L.ld_logits};
-  auto router = L.router_splits == 4   ? moe_router_gemm_kernel<4>
-                : L.router_splits == 2 ? moe_router_gemm_kernel<2>
-                                       : moe_router_gemm_kernel<1>;
-  hipLaunchKernelGGL(router, grid_for((T + kRtBM - 1) / kRtBM * router_blocks(E) * L.router_splits),
-                     dim3(64 * kRtWaves), kRtLds, st, r);
-  hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, r.part,
-                     L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
+  if (T <= kRsMaxTokens) {
+    hipLaunchKernelGGL(moe_router_short_kernel,
+                       dim3((E + kRsRows) / kRsRows, 4, (T + kRsTokens - 1) / kRsTokens), dim3(256),
+                       kRsLds, st, r);
+  } else {
+    auto router = L.router_splits == 4   ? moe_router_gemm_kernel<4>
+                  : L.router_splits == 2 ? moe_router_gemm_kernel<2>
+                                         : moe_router_gemm_kernel<1>;
+    hipLaunchKernelGGL(router, grid_for((T + kRtBM - 1) / kRtBM * router_blocks(E) * L.router_splits),
+                       dim3(64 * kRtWaves), kRtLds, st, r);
+  }
+  if (T <= kFewTokens)
+    hipLaunchKernelGGL(moe_topk_align_few_kernel, dim3(1), dim3(1024), 0, st, logits, r.part,
+                       L.router_splits, L.ld_logits, E, T, ids, rw, sgw, meta, sorted);
+  else
+    hipLaunchKernelGGL(moe_topk_kernel, dim3(tok_blocks), dim3(256), 0, st, logits, r.part,
+                       L.router_splits, L.ld_logits, E, T, ids, rw, sgw);
 
   StreamArgs a{h2, static_cast<const bf16*>(expert_gate_up), win + (size_t)(E + 1) * kMoeHidden,
                meta, sorted, rw, act, T, E, 1u};
   StreamArgs d{act, static_cast<const bf16*>(expert_down), static_cast<const bf16*>(shared_down),
                meta, sorted, rw, y, T, E, 1u};
   if (T <= kStreamMaxTokens) {
-    hipLaunchKernelGGL(moe_align_one_kernel, dim3(1), dim3(1024), 0, st, ids, T, E, meta, sorted);
+    if (T > kFewTokens)
+      hipLaunchKernelGGL(moe_align_one_kernel, dim3(1), dim3(1024), 0, st, ids, T, E, meta, sorted);
     hipLaunchKernelGGL(moe_stream_kernel<false>, grid_for(L.max_tiles * kStGateUpBlocks), dim3(512),
                        kStLds, st, a);
     d.subs = stream_down_subs(T);

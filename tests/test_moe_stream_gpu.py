@@ -18,6 +18,8 @@ TOL = 2e-2   # the block's output tolerance (bf16 roundings of each expert's row
     (12, 70),                    # uneven groups around one tile
     (256, 2), (256, 16),         # few experts, one row each
     (64, 64), (64, 65),          # one and two column blocks per down workgroup
+    (256, 17), (32, 512), (32, 513),   # alignment in two launches; router forms
+    (256, 63), (252, 66),        # router rows and tokens past the tiles' ends
 ])
 def test_stream_tile_edges(gpu, n_experts, tokens):
     from qwen36_attn.moe import MoEBlock
