@@ -47,7 +47,8 @@ constexpr int kVLds = kDecWaves * kDecBlock * kVPitch;   // 69632 bytes
 constexpr int kQPitch = 528;           // LDS row pitch of the Q^T operand
 constexpr int kKPitch = 528;           // LDS row pitch of the staged K rows
 constexpr int kKLds = kDecWaves * kDecBlock * kKPitch;   // 67584 bytes
-constexpr int kDecLds = kVLds + kKLds + 16 * kQPitch;    // 145664 bytes
+constexpr int kNewRow = kVLds + kKLds + 16 * kQPitch;    // the new K row, then V
+constexpr int kDecLds = kNewRow + 2 * kD * 2;            // 146688 bytes
 
 constexpr unsigned kMaxSplits = 256;
 // Default split count: 128 splits x 2 KV heads = one workgroup per CU.
@@ -113,13 +114,15 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
   const unsigned end = cache_end;
   // The workgroup that owns the new row's block writes the row into the
   // cache (this KV head's half: the copy of k_new / v_new, or in the fused
-  // step K after head norm and RoPE and V raw) and is its only reader, so it
-  // then streams that row from the cache like every other.  If the row lies
-  // in one of the first blocks (round < 4: short caches) the write completes
-  // before any load is issued; otherwise it overlaps the first loads and the
-  // workgroup barrier after Q staging orders it before the row's block is
-  // read.  Raw inputs of the fused step are requested before the first K/V
-  // block so that their (short) round trip does not queue behind it.
+  // step K after head norm and RoPE and V raw) and keeps it in LDS, where the
+  // wave that streams the block lays it over whatever its loads brought for
+  // that row, so no load waits for the row's store.  (It used to be written
+  // first and read back; for caches of up to four rounds of blocks that
+  // delayed the owner's loads by the norm and a store round trip: split +
+  // combine at 2051 tokens 14.2 us a layer, 13.3 now with the combine's
+  // unconditional loads; 128K unchanged.)  Raw inputs
+  // of the fused step are requested before the first K/V block so that their
+  // (short) round trip does not queue behind it.
   const bool owner = (position / kDecBlock) % nsplit == split;
   const bool new_row = owner && (kFuse || k_new != nullptr);
   float xq[2][4], xk[4];
@@ -139,6 +142,12 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
     }
     if (owner && wave == 1) vrow = *reinterpret_cast<const bf16x4*>(fz.v_raw + kvh * kD + 4 * lane);
   }
+  u32x4 nrow;   // k_new (lanes 0-31) or v_new, 16 bytes a lane
+  if constexpr (!kFuse) {
+    if (new_row && wave == 0)
+      nrow = reinterpret_cast<const u32x4*>((lane < 32 ? k_new : v_new) + kvh * kD)[lane & 31];
+  }
+  char* newrow = lds + kNewRow;
   auto write_new_row = [&]() {
     const size_t o = ((size_t)position * kHkv + kvh) * kD;
     if constexpr (kFuse) {
@@ -151,26 +160,16 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) yb[e] = f2bf(y[e]);
         *reinterpret_cast<bf16x4*>(k_cache + o + 4 * lane) = yb;
+        *reinterpret_cast<bf16x4*>(newrow + 8 * lane) = yb;
       } else if (wave == 1) {
         *reinterpret_cast<bf16x4*>(v_cache + o + 4 * lane) = vrow;
+        *reinterpret_cast<bf16x4*>(newrow + 2 * kD + 8 * lane) = vrow;
       }
     } else if (wave == 0) {
-      if (lane < 32) {
-        reinterpret_cast<uint4*>(k_cache + o)[lane] =
-            reinterpret_cast<const uint4*>(k_new + kvh * kD)[lane];
-      } else {
-        reinterpret_cast<uint4*>(v_cache + o)[lane - 32] =
-            reinterpret_cast<const uint4*>(v_new + kvh * kD)[lane - 32];
-      }
+      reinterpret_cast<u32x4*>((lane < 32 ? k_cache : v_cache) + o)[lane & 31] = nrow;
+      reinterpret_cast<u32x4*>(newrow)[lane] = nrow;
     }
   };
-  const bool early_row = new_row && (position / kDecBlock) / nsplit < (unsigned)kDecWaves;
-  if (early_row) {
-    write_new_row();
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-
 
   f32x4 o[16];
 #pragma unroll
@@ -233,8 +232,7 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
   // dims s*32 + 8*lg .. +8, so one K load instruction reads 16 rows x 64
   // contiguous bytes.
   char* qs = lds + kVLds + kKLds;
-  const bool late_row = new_row && !early_row;
-  if (late_row) write_new_row();
+  if (new_row) write_new_row();
   if constexpr (kFuse) {
     // Head norm + RoPE of this group's 8 query heads (wave w: heads 2w,
     // 2w+1) straight into the Q^T operand rows; rows 8..15 are zero padding.
@@ -265,9 +263,7 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
     *reinterpret_cast<uint4*>(qs + r * kQPitch + c * 16) = a;
     *reinterpret_cast<uint4*>(qs + r * kQPitch + (c + 16) * 16) = b;
   }
-  // the new row's stores complete before the barrier (the waves that wrote)
-  if (late_row && wave < 2) __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
+  lds_barrier();   // Q^T and the new row are in LDS; the block's loads stay in flight
   const char* qrow = qs + li * kQPitch + lg * 16;
   const char* krow0 = kbuf + li * kKPitch + lg * 16;
   for (; t0 < end; t0 += stride) {
@@ -275,6 +271,10 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
     // K of this block into the operand layout; the next block's K is then
     // requested at once (its registers are free)
     stage_k();
+    const bool lay_new = new_row && position - t0 < (unsigned)kDecBlock;   // wave-uniform
+    if (lay_new && lane < 32)
+      *reinterpret_cast<u32x4*>(kbuf + (position - t0) * kKPitch + lane * 16) =
+          *reinterpret_cast<const u32x4*>(newrow + lane * 16);
     if (tn < end) load_k(tn);
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -318,6 +318,9 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
       *reinterpret_cast<u32x4*>(vbuf + (2 * c + (lane >> 5)) * kVPitch +
                                 (lane & 31) * 16) = vr[c];
     }
+    if (lay_new && lane < 32)
+      *reinterpret_cast<u32x4*>(vbuf + (position - t0) * kVPitch + lane * 16) =
+          *reinterpret_cast<const u32x4*>(newrow + 2 * kD + lane * 16);
     if (tn < end) load_v(tn);
     bf16x8 pb;
 #pragma unroll
@@ -380,13 +383,15 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
 // workgroups.  Every load (the split partials, their (m, l), the gate) is
 // issued up front: one memory round trip.
 constexpr int kCombineDims = 16;
-static_assert(kMaxSplits % 16 == 0, "16 split groups per combine wave");
 
 // Lane = (split group sg = lane / 4, dim quad dq = lane % 4); split group sg
 // takes splits sg, sg + 16, ...  The max, the weights 2^(m - M) and the sums
 // reduce over the 16 split groups with xor shuffles (lane bits 2..5): no LDS,
 // no barrier.  Measured on MI355X against a 4-wave combine with LDS
-// reductions: -0.2 to -0.7 us per layer.
+// reductions: -0.2 to -0.7 us per layer.  kPer = splits per group (the least
+// power of two that covers nsplit); every load is unconditional at a clamped
+// index and masked afterwards.
+template <int kPer>
 __global__ __launch_bounds__(64) void decode_gqa_combine_wave_kernel(
     const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
     unsigned nsplit, const bf16* __restrict__ gate, unsigned gate_head_stride,
@@ -397,19 +402,13 @@ __global__ __launch_bounds__(64) void decode_gqa_combine_wave_kernel(
   const int dq = lane & 3, sg = lane >> 2;
   const int d0 = (blockIdx.x >> 4) * kCombineDims + 4 * dq;
   const size_t base = (size_t)kvh * nsplit * kGroup + hh;
-  constexpr int kPer = kMaxSplits / 16;   // at most 16 splits per group
   float2 ml[kPer];
   f32x4 os[kPer];
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
-    const unsigned sp = sg + 16 * u;
-    if (sp < nsplit) {
-      ml[u] = *reinterpret_cast<const float2*>(ws_ml + (base + (size_t)sp * kGroup) * 2);
-      os[u] = *reinterpret_cast<const f32x4*>(ws_o + (base + (size_t)sp * kGroup) * kD + d0);
-    } else {
-      ml[u] = float2{-INFINITY, 0.f};
-      os[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    const size_t at = base + (size_t)min(sg + 16u * u, nsplit - 1) * kGroup;
+    ml[u] = *reinterpret_cast<const float2*>(ws_ml + at * 2);
+    os[u] = *reinterpret_cast<const f32x4*>(ws_o + at * kD + d0);
   }
   // the gate is requested after the partials (and every lane reads it, kept
   // as raw bits), so its load joins their round trip instead of preceding it
@@ -420,7 +419,13 @@ __global__ __launch_bounds__(64) void decode_gqa_combine_wave_kernel(
   }
   float mx = -INFINITY;
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) mx = fmaxf(mx, ml[u].x);
+  for (int u = 0; u < kPer; ++u) {
+    if (sg + 16u * u >= nsplit) {
+      ml[u] = float2{-INFINITY, 0.f};
+      os[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    mx = fmaxf(mx, ml[u].x);
+  }
   mx = wave_max_xor(mx, 4);
   mx = wave_max_xor(mx, 8);
   mx = wave_max_xor(mx, 16);
@@ -515,7 +520,13 @@ static int launch_decode(bool fuse, const void* q, const void* k_new,
                      static_cast<bf16*>(v_cache), static_cast<const bf16*>(k_new),
                      static_cast<const bf16*>(v_new), position, cache_end, nsplit, ws,
                      fz);
-  hipLaunchKernelGGL(decode_gqa_combine_wave_kernel, dim3(kHq * (kD / kCombineDims)), dim3(64),
+  static_assert(kMaxSplits == 16 * 16, "combine forms");
+  auto combine = nsplit <= 16   ? decode_gqa_combine_wave_kernel<1>
+                 : nsplit <= 32 ? decode_gqa_combine_wave_kernel<2>
+                 : nsplit <= 64 ? decode_gqa_combine_wave_kernel<4>
+                 : nsplit <= 128 ? decode_gqa_combine_wave_kernel<8>
+                                 : decode_gqa_combine_wave_kernel<16>;
+  hipLaunchKernelGGL(combine, dim3(kHq * (kD / kCombineDims)), dim3(64),
                      0, st, ws.o, ws.ml, nsplit, static_cast<const bf16*>(gate),
                      gate_head_stride, static_cast<bf16*>(out));
   return static_cast<int>(hipGetLastError());
