@@ -145,6 +145,40 @@ __device__ __forceinline__ bf16x8 cat_bf16x8(i16x4 lo, i16x4 hi) {
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// What one workgroup of the 4096-wide GEMV reads (8 rows of 8 KiB), and the most
+// that a launch reads ahead for the next (the L2s together hold 32 MiB).
+constexpr int kWarmPiece = 65536;
+constexpr size_t kWarmMax = (size_t)32 << 20;
+
+// Reads `bytes` at p (16-byte aligned) and drops them, so that they are in this
+// XCD's L2 when the launch behind asks: for workgroups of a latency-bound
+// launch that have nothing else to do, over weights that the next launch
+// streams.  Workgroup j of n (n a multiple of 8) takes pieces j, j + n, ... of
+// kPiece bytes; where the next launch's workgroup b reads piece b and both
+// launches deal workgroups to the 8 XCDs in turn, the lines land in the L2
+// that asks for them.  Purely a hint: nothing is written, and loads past
+// `bytes` are dropped by the buffer range.
+template <int kPiece, int kThreads>
+__device__ __forceinline__ void warm_l2(const void* p, unsigned bytes, unsigned j, unsigned n) {
+  constexpr unsigned kSlice = kThreads * 16, kPer = kPiece / kSlice;
+  static_assert(kPiece % kSlice == 0, "whole slices");
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+  const unsigned pieces = (bytes + kPiece - 1) / kPiece;
+  const unsigned slices = j < pieces ? (pieces - j + n - 1) / n * kPer : 0;
+  for (unsigned s0 = 0; s0 < slices; s0 += 8) {
+    u32x4 x[8];
+#pragma unroll
+    for (unsigned u = 0; u < 8; ++u) {
+      const unsigned s = s0 + u;
+      x[u] = __builtin_amdgcn_raw_buffer_load_b128(
+          rs, (int)((j + s / kPer * n) * kPiece + s % kPer * kSlice + threadIdx.x * 16), 0, 0);
+    }
+#pragma unroll
+    for (unsigned u = 0; u < 8; ++u) asm volatile("" ::"v"(x[u]));
+  }
+}
+
 // Workgroup barrier for LDS traffic only: waits for this wave's LDS operations
 // (lgkmcnt) but, unlike __syncthreads(), not for its outstanding global loads,
 // so prefetches stay in flight across the barrier.  The signal fences keep

@@ -56,6 +56,14 @@ constexpr unsigned kMaxSplits = 256;
 // -- and 64..192; one workgroup holding both KV heads was no faster.)
 constexpr unsigned kTargetSplits = 128;
 
+// Up to 128 split workgroups at least half of the CUs are idle during the split
+// launch (each workgroup's LDS fills a CU): where the caller names what the
+// launch after the combine streams (o_proj, 16.8 MB), as many more workgroups
+// read it into L2 meanwhile.  From 4097 cached tokens on they only compete with
+// the K and V stream.  MI355X, us a layer with projections, without / with: 400
+// rows 25.2 / 24.7, 2051 25.2 / 24.9, 6000 25.9 / 26.1, 8192 26.5 / 27.1.
+constexpr unsigned kDecWarmGroups = 128, kDecWarmEnd = 4096;
+
 // RoPE inverse frequencies for the fused decode step (this translation
 // unit's copy; see rope_inv_freq_host).
 __constant__ float c_dec_inv_freq[kRotaryPairs];
@@ -93,7 +101,15 @@ __global__ __launch_bounds__(256, 1) void decode_gqa_split_kernel(
     const bf16* __restrict__ q, bf16* __restrict__ k_cache,
     bf16* __restrict__ v_cache, const bf16* __restrict__ k_new,
     const bf16* __restrict__ v_new, unsigned position, unsigned cache_end,
-    unsigned nsplit, DecodeWs ws, FuseArgs fz) {
+    unsigned nsplit, DecodeWs ws, FuseArgs fz, const void* next, unsigned next_bytes) {
+  if constexpr (kFuse) {
+    if (blockIdx.x >= nsplit * kHkv) {
+      const unsigned first = (nsplit * kHkv + 7) & ~7u;
+      if (blockIdx.x >= first)
+        warm_l2<kWarmPiece, 256>(next, next_bytes, blockIdx.x - first, kDecWarmGroups);
+      return;
+    }
+  }
   __shared__ __attribute__((aligned(16))) char lds[kDecLds];
   // Workgroup i streams KV head i % 2: consecutive workgroups are dealt to
   // the 8 XCDs in turn, so each XCD serves one head (the half of every
@@ -505,7 +521,7 @@ static int launch_decode(bool fuse, const void* q, const void* k_new,
                          unsigned capacity, const void* gate,
                          unsigned gate_head_stride, void* out, void* workspace,
                          size_t workspace_bytes_given, unsigned split_tokens,
-                         void* stream) {
+                         const void* next, size_t next_bytes, void* stream) {
   const unsigned per = split_tokens ? split_tokens : choose_split_tokens(cache_end);
   const unsigned nsplit = (cache_end + per - 1) / per;
   if (nsplit > kMaxSplits) return Q36_EINVAL;
@@ -515,11 +531,15 @@ static int launch_decode(bool fuse, const void* q, const void* k_new,
   ws.ml = ws.o + (size_t)nsplit * kHkv * kGroup * kD;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto kernel = fuse ? decode_gqa_split_kernel<true> : decode_gqa_split_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(nsplit * kHkv), dim3(256), 0, st,
+  const unsigned splits = nsplit * kHkv;
+  const unsigned grid = next != nullptr && splits <= kDecWarmGroups && cache_end <= kDecWarmEnd
+                            ? ((splits + 7) & ~7u) + kDecWarmGroups
+                            : splits;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, st,
                      static_cast<const bf16*>(q), static_cast<bf16*>(k_cache),
                      static_cast<bf16*>(v_cache), static_cast<const bf16*>(k_new),
                      static_cast<const bf16*>(v_new), position, cache_end, nsplit, ws,
-                     fz);
+                     fz, next, (unsigned)next_bytes);
   static_assert(kMaxSplits == 16 * 16, "combine forms");
   auto combine = nsplit <= 16   ? decode_gqa_combine_wave_kernel<1>
                  : nsplit <= 32 ? decode_gqa_combine_wave_kernel<2>
@@ -581,17 +601,18 @@ Q36_EXPORT int qwen36_decode_gqa(const void* q, const void* k_new,
     return Q36_EINVAL;
   return launch_decode(false, q, k_new, v_new, FuseArgs{}, k_cache, v_cache, position,
                        cache_end, capacity, gate, gate_head_stride, out, workspace,
-                       workspace_bytes_given, split_tokens, stream);
+                       workspace_bytes_given, split_tokens, nullptr, 0, stream);
 }
 
-Q36_EXPORT int qwen36_decode_step(const void* q_gate, const void* k_raw,
-                                  const void* v_raw, const void* q_norm_weight,
-                                  const void* k_norm_weight, void* k_cache,
-                                  void* v_cache, unsigned position,
-                                  unsigned cache_end, unsigned capacity,
-                                  void* out, void* workspace,
-                                  size_t workspace_bytes_given,
-                                  unsigned split_tokens, void* stream) {
+Q36_EXPORT int qwen36_decode_step_next(const void* q_gate, const void* k_raw,
+                                       const void* v_raw, const void* q_norm_weight,
+                                       const void* k_norm_weight, void* k_cache,
+                                       void* v_cache, unsigned position,
+                                       unsigned cache_end, unsigned capacity,
+                                       void* out, void* workspace,
+                                       size_t workspace_bytes_given,
+                                       unsigned split_tokens, const void* next_weight,
+                                       size_t next_bytes, void* stream) {
   if (q_gate == nullptr || k_raw == nullptr || v_raw == nullptr ||
       q_norm_weight == nullptr || k_norm_weight == nullptr || k_cache == nullptr ||
       v_cache == nullptr || out == nullptr || workspace == nullptr || cache_end == 0 ||
@@ -601,7 +622,9 @@ Q36_EXPORT int qwen36_decode_step(const void* q_gate, const void* k_raw,
       (reinterpret_cast<uintptr_t>(k_raw) % 8) != 0 ||
       (reinterpret_cast<uintptr_t>(v_raw) % 8) != 0 ||
       (reinterpret_cast<uintptr_t>(k_cache) % 8) != 0 ||
-      (reinterpret_cast<uintptr_t>(v_cache) % 8) != 0)
+      (reinterpret_cast<uintptr_t>(v_cache) % 8) != 0 ||
+      (next_weight == nullptr) != (next_bytes == 0) || next_bytes > kWarmMax ||
+      (reinterpret_cast<uintptr_t>(next_weight) % 16) != 0)
     return Q36_EINVAL;
   const int st = ensure_dec_inv_freq();
   if (st != Q36_OK) return st;
@@ -614,7 +637,21 @@ Q36_EXPORT int qwen36_decode_step(const void* q_gate, const void* k_raw,
   // The gate is the second half of each head's 512-wide q-projection slice.
   return launch_decode(true, nullptr, nullptr, nullptr, fz, k_cache, v_cache, position,
                        cache_end, capacity, static_cast<const bf16*>(q_gate) + kD, 2 * kD,
-                       out, workspace, workspace_bytes_given, split_tokens, stream);
+                       out, workspace, workspace_bytes_given, split_tokens, next_weight,
+                       next_bytes, stream);
+}
+
+Q36_EXPORT int qwen36_decode_step(const void* q_gate, const void* k_raw,
+                                  const void* v_raw, const void* q_norm_weight,
+                                  const void* k_norm_weight, void* k_cache,
+                                  void* v_cache, unsigned position,
+                                  unsigned cache_end, unsigned capacity,
+                                  void* out, void* workspace,
+                                  size_t workspace_bytes_given,
+                                  unsigned split_tokens, void* stream) {
+  return qwen36_decode_step_next(q_gate, k_raw, v_raw, q_norm_weight, k_norm_weight, k_cache,
+                                 v_cache, position, cache_end, capacity, out, workspace,
+                                 workspace_bytes_given, split_tokens, nullptr, 0, stream);
 }
 
 Q36_EXPORT int qwen36_decode_gqa_noalloc(const void* q, const void* k_new,
@@ -638,5 +675,5 @@ Q36_EXPORT int qwen36_decode_gqa_noalloc(const void* q, const void* k_new,
   if (st != Q36_OK) return st;
   return launch_decode(false, q, k_new, v_new, FuseArgs{}, k_cache, v_cache, position,
                        cache_end, capacity, gate, gate_head_stride, out, ws, kScratchBytes,
-                       split_tokens, stream);
+                       split_tokens, nullptr, 0, stream);
 }

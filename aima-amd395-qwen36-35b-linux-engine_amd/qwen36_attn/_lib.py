@@ -42,6 +42,8 @@ SIGNATURES: dict[str, tuple] = {
                                          _vp, _u32, _vp, _u32, _vp]),
     "qwen36_decode_step": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32,
                                   _vp, _vp, _sz, _u32, _vp]),
+    "qwen36_decode_step_next": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32,
+                                       _vp, _vp, _sz, _u32, _vp, _sz, _vp]),
     # pointwise (full attention)
     "qwen36_rotary_table": (_i32, [_vp, _vp, _u32, _u32, _vp]),
     "qwen36_head_norm_rope": (_i32, [_vp, _u32, _vp, _u32, _vp, _u32, _vp, _vp,
@@ -91,6 +93,9 @@ SIGNATURES: dict[str, tuple] = {
     "qwen36_prefix_cache_destroy": (_i32, [_vp]),
     "qwen36_gdn_decode_step": (_i32, [_vp, _u32, _vp, _vp, _vp, _vp, _vp, _u32, _vp,
                                       _vp, _vp, _u32, _vp, _vp, _vp, _vp, _u32, _vp]),
+    "qwen36_gdn_decode_step_next": (_i32, [_vp, _u32, _vp, _vp, _vp, _vp, _vp, _u32, _vp,
+                                           _vp, _vp, _u32, _vp, _vp, _vp, _vp, _u32, _vp, _sz,
+                                           _vp]),
 }
 
 _LIB = None

@@ -27,6 +27,20 @@ def require(t: torch.Tensor, name: str, dtype: torch.dtype, shape=None,
         raise ValueError(f"{name} must be contiguous")
 
 
+_READ_AHEAD_MAX = 32 << 20   # the L2s together; the C entries refuse more
+
+
+def read_ahead(t: torch.Tensor | None, device: torch.device) -> tuple[int | None, int]:
+    """(address, bytes) of a tensor that the next launch streams, as the entries
+    with a ``next_weight`` take them.  Only a hint: whatever they would refuse
+    (and the launch that reads the tensor may yet accept or refuse itself) is
+    left out."""
+    if (not isinstance(t, torch.Tensor) or t.device != device or not t.is_contiguous()
+            or t.data_ptr() % 16 or not 0 < t.nbytes <= _READ_AHEAD_MAX):
+        return None, 0
+    return t.data_ptr(), t.nbytes
+
+
 _SCRATCH: dict[tuple[str, int], torch.Tensor] = {}
 # Buffers replaced by a larger one stay allocated: a HIP graph captured
 # earlier may still hold their addresses, and freeing them would let the

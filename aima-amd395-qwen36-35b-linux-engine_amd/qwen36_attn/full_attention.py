@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._tensors import ptr, require, scratch, stream_handle
+from ._tensors import ptr, read_ahead, require, scratch, stream_handle
 
 HQ, HKV, HEAD_DIM = 16, 2, 256
 Q_DIM, KV_DIM = HQ * HEAD_DIM, HKV * HEAD_DIM
@@ -85,7 +85,8 @@ def decode_gqa(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
 def decode_step(q_gate: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                 q_norm: torch.Tensor, k_norm: torch.Tensor, k_cache: torch.Tensor,
                 v_cache: torch.Tensor, position: int, cache_end: int | None = None,
-                out: torch.Tensor | None = None, split_tokens: int = 0) -> torch.Tensor:
+                out: torch.Tensor | None = None, split_tokens: int = 0,
+                next_weight: torch.Tensor | None = None) -> torch.Tensor:
     """The whole one-token decode of the gated full-attention layer between
     its projections and o_proj (four_layer_mini_engine.py:6546-6653, mode
     "decode") in one fused split launch plus the combine: head norm + RoPE
@@ -93,7 +94,9 @@ def decode_step(q_gate: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     raw), split-K attention over rows [0, cache_end) and the sigmoid output
     gate.  q_gate [1, 8192] (or [8192]) is the fused q projection row; k, v
     [1, 512] raw; returns [1, 4096] bf16.  Same rounding as
-    ``head_norm_rope_kv_write`` followed by ``decode_gqa``."""
+    ``head_norm_rope_kv_write`` followed by ``decode_gqa``.  ``next_weight``
+    (o_proj): what the next launch streams, read into L2 by CUs that the split
+    leaves idle; the results are the same."""
     dev = q_gate.device
     if cache_end is None:
         cache_end = position + 1
@@ -113,12 +116,12 @@ def decode_step(q_gate: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if out is None:
         out = torch.empty(1, Q_DIM, dtype=torch.bfloat16, device=dev)
     require(out, "out", torch.bfloat16)
-    lib = _lib.load(("qwen36_decode_step",))
+    lib = _lib.load(("qwen36_decode_step_next",))
     ws_bytes = lib.qwen36_decode_gqa_workspace_bytes(cache_end, split_tokens)
     ws = scratch("decode_gqa", ws_bytes, dev)
-    _lib.call("qwen36_decode_step", ptr(q_gate), ptr(k), ptr(v), ptr(q_norm), ptr(k_norm),
+    _lib.call("qwen36_decode_step_next", ptr(q_gate), ptr(k), ptr(v), ptr(q_norm), ptr(k_norm),
               ptr(k_cache), ptr(v_cache), position, cache_end, capacity, ptr(out), ptr(ws),
-              ws.numel(), split_tokens, stream_handle(dev))
+              ws.numel(), split_tokens, *read_ahead(next_weight, dev), stream_handle(dev))
     return out
 
 
@@ -333,7 +336,8 @@ class FullAttentionLayer:
                 self._qkv = FusedProjection(w["q_proj"], w["k_proj"], w["v_proj"])
             q_gate, k, v = self._qkv(inp)
             attn = decode_step(q_gate, k, v, w["q_norm"], w["k_norm"], self.k_cache,
-                               self.v_cache, position_start, cache_end)
+                               self.v_cache, position_start, cache_end,
+                               next_weight=w["o_proj"])
             from .projections import gemv
             return gemv(w["o_proj"], attn)
         from .prefill_gemm import linear

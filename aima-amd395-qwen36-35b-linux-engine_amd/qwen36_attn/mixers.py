@@ -166,7 +166,7 @@ def full_attention(inp: torch.Tensor, layer_index: int, weights: dict) -> torch.
         proj = st.fused_projection(layer_index, "qkv", w["q_proj"], w["k_proj"], w["v_proj"])
         q_gate, k, v = proj(inp)
         attn = fa.decode_step(q_gate, k, v, w["q_norm"], w["k_norm"], k_cache, v_cache,
-                              st.position_start, st.position_end)
+                              st.position_start, st.position_end, next_weight=w["o_proj"])
         return gemv(w["o_proj"], attn)
     cache_end = st.position_end if st.position_start > 0 else t
     proj = st.fused_projection(layer_index, "qkv", w["q_proj"], w["k_proj"], w["v_proj"])
@@ -210,7 +210,8 @@ def linear_attention(inp: torch.Tensor, layer_index: int, weights: dict) -> torc
     if st.mode == "decode":
         gated = gd.gdn_decode_step(mixed, conv_in, conv_out, cw, a, b, w["linear_A_log"],
                                    w["linear_dt_bias"], z, w["linear_norm"], ssm_in,
-                                   final_state=ssm_out)
+                                   final_state=ssm_out,
+                                   next_weight=w["linear_out_proj"] if t == 1 else None)
         return gemv(w["linear_out_proj"], gated) if t == 1 else pg.linear(gated, w["linear_out_proj"])
     conv, _ = gd.causal_conv1d(mixed, conv_in, cw, new_state=conv_out)
     q = conv[:, :gd.KEY_DIM].view(t, gd.HK, gd.DK)

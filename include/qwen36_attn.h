@@ -156,6 +156,18 @@ int qwen36_decode_step(const void* q_gate, const void* k_raw, const void* v_raw,
                        void* workspace, size_t workspace_bytes,
                        unsigned split_tokens, void* stream);
 
+/* qwen36_decode_step_next: the same, told what the next launch streams
+ * (o_proj: next_bytes at next_weight, 16-byte aligned, at most 32 MiB; null and
+ * 0 for nothing), so that CUs which the split leaves idle (up to 4096 cached
+ * tokens) read it into L2 meanwhile.  Same results; nothing is kept. */
+int qwen36_decode_step_next(const void* q_gate, const void* k_raw, const void* v_raw,
+                            const void* q_norm_weight, const void* k_norm_weight,
+                            void* k_cache, void* v_cache, unsigned position,
+                            unsigned cache_end, unsigned capacity, void* out,
+                            void* workspace, size_t workspace_bytes,
+                            unsigned split_tokens, const void* next_weight,
+                            size_t next_bytes, void* stream);
+
 /* ---- full-attention pointwise ----------------------------------------------
  * qwen36_rotary_table: replaces prefill_rotary_table_kernel /
  *   decode_rotary_kernel (native_pointwise.hip.cpp:224-238,
@@ -312,6 +324,18 @@ int qwen36_gdn_decode_step(const void* mixed_qkv, unsigned x_row_stride,
                            unsigned z_row_stride, const void* norm_weight,
                            const void* state_in, void* state_out, void* out,
                            unsigned tokens, void* stream);
+
+/* qwen36_gdn_decode_step_next: the same, told what the next launch streams
+ * (out_proj; see qwen36_decode_step_next). */
+int qwen36_gdn_decode_step_next(const void* mixed_qkv, unsigned x_row_stride,
+                                const void* conv_weight, const void* conv_state_in,
+                                void* conv_state_out, const void* a, const void* b,
+                                unsigned ab_row_stride, const void* a_log,
+                                const void* dt_bias, const void* z,
+                                unsigned z_row_stride, const void* norm_weight,
+                                const void* state_in, void* state_out, void* out,
+                                unsigned tokens, const void* next_weight,
+                                size_t next_bytes, void* stream);
 
 /* ---- prefill projections ---------------------------------------------------
  * qwen36_prefill_gemm_bf16: y[m, n] = x[m, k] W[n, k]^T for a prompt of m

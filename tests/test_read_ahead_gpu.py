@@ -1,0 +1,75 @@
+"""Decode steps told what the next launch streams: the workgroups that read it
+ahead change nothing, whatever its size (a ragged last piece, one 16-byte row,
+more pieces than workgroups) and whether or not the split leaves room for them
+(up to 128 split workgroups), and the hint never refuses a call."""
+import pytest
+import torch
+
+from qwen36_attn import synthetic as syn
+from tests.test_gdn_decode_step_gpu import _step_inputs
+
+BF16 = torch.bfloat16
+ELEMENTS = [8, 32768 + 24, 2048 * 4096, 16 << 20]
+
+
+def test_read_ahead_hint_is_optional():
+    from qwen36_attn._tensors import read_ahead
+    dev = torch.device("cpu")
+    x = torch.zeros(64, 8, dtype=BF16)
+    assert read_ahead(x, dev) == (x.data_ptr(), 1024)
+    for t in (None, x.t(), x[:0], x.view(-1)[4:], "o_proj", x.to("meta"),
+              torch.empty((16 << 20) + 8, dtype=BF16)):
+        assert read_ahead(t, dev) == (None, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elements", ELEMENTS)
+@pytest.mark.parametrize("rows,split", [(1, 0), (2051, 0), (8192, 0), (8193, 0), (8192, 128)])
+def test_attention_step_with_next_weight(gpu, rows, split, elements):
+    from qwen36_attn.full_attention import decode_step
+    g = syn.gen(rows)
+    q, k, v = (syn.randn((1, n), g).to(gpu) for n in (8192, 512, 512))
+    qw, kw = (syn.randn((256,), g, 0.1).to(gpu) for _ in range(2))
+    kc, vc = (syn.randn((rows, 2, 256), g).to(gpu) for _ in range(2))
+    kc2, vc2 = kc.clone(), vc.clone()
+    w = syn.randn((elements,), syn.gen(1)).to(gpu)
+    w0 = w.clone()
+    print(f"decode step rows={rows} split={split} next={elements}", flush=True)
+    got = decode_step(q, k, v, qw, kw, kc, vc, rows - 1, split_tokens=split, next_weight=w)
+    want = decode_step(q, k, v, qw, kw, kc2, vc2, rows - 1, split_tokens=split)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    assert torch.equal(w, w0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elements", ELEMENTS)
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_gdn_step_with_next_weight(gpu, tokens, elements):
+    from qwen36_attn.gated_deltanet import gdn_decode_step
+    mixed, conv_w, conv, a, b, a_log, dt, z, nw, ssm = (
+        x.to(gpu) for x in _step_inputs(tokens, 7, 1.0))
+    w = syn.randn((elements,), syn.gen(2)).to(gpu)
+    w0 = w.clone()
+    print(f"gdn step tokens={tokens} next={elements}", flush=True)
+    outs = []
+    for nxt in (w, None):
+        new_conv, state = torch.empty_like(conv), torch.empty_like(ssm)
+        out = gdn_decode_step(mixed, conv, new_conv, conv_w, a, b, a_log, dt, z, nw, ssm,
+                              final_state=state, next_weight=nxt)
+        outs.append((out, new_conv, state))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
+    assert torch.equal(w, w0)
+
+
+def test_next_weight_refusals():
+    """C entries: bytes without an address, an address without bytes, more than
+    the L2s hold, an address off 16 bytes."""
+    from qwen36_attn import _lib
+    L = _lib.load(("qwen36_decode_step_next", "qwen36_gdn_decode_step_next"))
+    for nxt in ((None, 16), (32, 0), (32, (32 << 20) + 1), (40, 16)):
+        assert L.qwen36_decode_step_next(16, 16, 16, 16, 16, 16, 16, 0, 1, 1, 16, 16, 1 << 30, 0,
+                                         *nxt, None) == 1
+        assert L.qwen36_gdn_decode_step_next(16, 8192, 32, 4096, 1 << 20, 48, 64, 32, 80, 96, 128,
+                                             4096, 160, 256, 256, 512, 1, *nxt, None) == 1
