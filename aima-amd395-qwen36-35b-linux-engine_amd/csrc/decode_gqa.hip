@@ -61,7 +61,8 @@ constexpr unsigned kTargetSplits = 128;
 // launch after the combine streams (o_proj, 16.8 MB), as many more workgroups
 // read it into L2 meanwhile.  From 4097 cached tokens on they only compete with
 // the K and V stream.  MI355X, us a layer with projections, without / with: 400
-// rows 25.2 / 24.7, 2051 25.2 / 24.9, 6000 25.9 / 26.1, 8192 26.5 / 27.1.
+// rows 23.6 / 22.7, 2051 24.1 / 23.6, 4096 24.9 / 24.5, 6000 25.5 / 25.9, 8192
+// 26.5 / 27.1.
 constexpr unsigned kDecWarmGroups = 128, kDecWarmEnd = 4096;
 
 // RoPE inverse frequencies for the fused decode step (this translation
@@ -475,15 +476,27 @@ __global__ __launch_bounds__(64) void decode_gqa_combine_wave_kernel(
   }
 }
 
-unsigned choose_split_tokens(unsigned cache_end) {
-  // Aim for one workgroup per CU (256 CUs) over both KV heads while keeping
-  // at least one 32-token block per wave.
-  const unsigned target_splits = kTargetSplits;
-  unsigned per = (cache_end + target_splits - 1) / target_splits;
+// Long caches: one workgroup per CU (256 CUs) over both KV heads, with at least
+// one 32-token block per wave.  Up to 8192 tokens the call is a latency chain
+// and a workgroup's share its longest link, so the cache goes to at most 64
+// splits (128 workgroups) of any number of blocks; a wave without a block waits
+// at the merge.  MI355X, projections + split + combine, us a layer, splits of
+// 32 / 64 / 96 / 128 tokens: 400 rows 22.7 / 23.1 / 24.0 / 24.7, 1000 23.1 / 23.3
+// / 24.1 / 24.8, 2051 24.1 / 23.6 / 24.4 / 24.9, 4096 25.6 / 24.5 / 25.6 / 25.7,
+// 6000 32.2 (more workgroups than CUs) / 25.6 / 25.5 / 25.9, 8192 33.3 / 26.6 /
+// 26.5 / 26.5; 12000 with 96 or 128 27.9.
+constexpr unsigned kFineEnd = 8192, kFineSplits = 64;
+
+unsigned coarse_split_tokens(unsigned cache_end) {
+  const unsigned per = (cache_end + kTargetSplits - 1) / kTargetSplits;
   const unsigned quantum = kDecWaves * kDecBlock;  // 128
-  per = (per + quantum - 1) / quantum * quantum;
-  if (per < quantum) per = quantum;
-  return per;
+  return (per + quantum - 1) / quantum * quantum;
+}
+
+unsigned choose_split_tokens(unsigned cache_end) {
+  if (cache_end > kFineEnd) return coarse_split_tokens(cache_end);
+  const unsigned per = (cache_end + kFineSplits - 1) / kFineSplits;
+  return (per + kDecBlock - 1) / kDecBlock * kDecBlock;
 }
 
 size_t workspace_bytes(unsigned nsplit) {
@@ -511,6 +524,9 @@ using namespace q36;
 Q36_EXPORT size_t qwen36_decode_gqa_workspace_bytes(unsigned cache_end,
                                                     unsigned split_tokens) {
   if (cache_end == 0) return 0;
+  // one size for the short caches: their split count is not monotonic (it falls
+  // where the split size steps up), so a buffer serves all of them
+  if (split_tokens == 0 && cache_end <= kFineEnd) return workspace_bytes(kFineSplits);
   const unsigned per = split_tokens ? split_tokens : choose_split_tokens(cache_end);
   return workspace_bytes((cache_end + per - 1) / per);
 }
@@ -522,7 +538,10 @@ static int launch_decode(bool fuse, const void* q, const void* k_new,
                          unsigned gate_head_stride, void* out, void* workspace,
                          size_t workspace_bytes_given, unsigned split_tokens,
                          const void* next, size_t next_bytes, void* stream) {
-  const unsigned per = split_tokens ? split_tokens : choose_split_tokens(cache_end);
+  unsigned per = split_tokens ? split_tokens : choose_split_tokens(cache_end);
+  // a caller's smaller workspace takes the fewer splits that it has room for
+  if (split_tokens == 0 && workspace_bytes_given < workspace_bytes((cache_end + per - 1) / per))
+    per = coarse_split_tokens(cache_end);
   const unsigned nsplit = (cache_end + per - 1) / per;
   if (nsplit > kMaxSplits) return Q36_EINVAL;
   if (workspace_bytes_given < workspace_bytes(nsplit)) return Q36_EINVAL;
