@@ -79,6 +79,7 @@ struct SplitArgs {
   float* ml;            // [tile][chunk][kv head][rows][2]
   unsigned chunk_keys;  // multiple of 32
   unsigned n_chunks;
+  unsigned ranges;      // items dealt to the XCDs as contiguous ranges
 };
 
 // Gated output (kGate): out_bf16[row][h*256 + d] = gate_bf16(O, gate[row *
@@ -90,27 +91,33 @@ struct GateArgs {
   bf16* out;
 };
 
-template <int kFmWaves, bool kSplit, bool kGate = false>
-__global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_prefill_kernel(
+// kSub = 2: two groups of kFmWaves waves share the tile's rows, each with an LDS
+// ring of its own and half of the chunk's keys, and merge in LDS at the end, so
+// the workgroup writes one partial of half as many rows as 2 kFmWaves waves of
+// rows would, for the same keys per wave.
+template <int kFmWaves, bool kSplit, bool kGate = false, int kSub = 1>
+__global__ __launch_bounds__(64 * kFmWaves * kSub, kFmWaves * kSub == 8 ? 1 : 2) void fmha_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k,
     const bf16* __restrict__ v, float* __restrict__ out, unsigned q_tokens,
     unsigned kv_tokens, unsigned n_qtiles, SplitArgs sp, GateArgs ga) {
   static_assert(!(kSplit && kGate), "split partials are gated by the combine");
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  static_assert(kSub == 1 || (kSub == 2 && kSplit), "the split form merges pairs");
+  extern __shared__ __attribute__((aligned(1024))) char lds_all[];
   constexpr int kFmRows = kFmWaves * kFmRowsPerWave;
   constexpr unsigned kTok = kFmRows / kGroup;          // tokens per tile
   constexpr int kFmLoadsPerWave = 16 / kFmWaves;       // 16 row-pair blocks per tile
 
   // XCD-aware tile mapping (see header).  Split: the (chunk, tile) items of a
   // KV head, chunk by chunk and heaviest tile first, are dealt to its four
-  // XCDs in turn (contiguous ranges, so that a chunk's rows go to one L2,
-  // measured no faster: 1000 rows over 4096 96 us against 90).
+  // XCDs in turn, or as contiguous ranges so that the few tiles of a long
+  // chunk read its keys through one L2 (see split_plan).
   const unsigned b = blockIdx.x, n = b >> 3, x4 = b & 3;
   const int kvh = (b >> 2) & 1;
   unsigned qtile, chunk = 0;
   if constexpr (kSplit) {
-    const unsigned i = 4 * n + x4;
-    if (i >= n_qtiles * sp.n_chunks) return;
+    const unsigned items = n_qtiles * sp.n_chunks, share = (items + 3) / 4;
+    const unsigned i = sp.ranges ? x4 * share + n : 4 * n + x4;
+    if (i >= items) return;
     chunk = i / n_qtiles;
     qtile = n_qtiles - 1 - i % n_qtiles;
   } else {
@@ -120,7 +127,10 @@ __global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_pre
   const unsigned tok0 = qtile * kTok;
 
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wave = kSub == 1 ? wave_wg : wave_wg % kFmWaves;
+  const int sub = kSub == 1 ? 0 : wave_wg / kFmWaves;
+  char* lds = lds_all + sub * kFmLds;
   const int lj = lane & 31;     // MFMA column (query row within the wave)
   const int lg = lane >> 5;     // k-half
   const unsigned off = kv_tokens - q_tokens;   // bottom-right shift
@@ -135,10 +145,13 @@ __global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_pre
   const unsigned wave_lim =
       min(wave_first + kFmRowsPerWave / kGroup - 1, q_tokens - 1) + off;
   const unsigned kv_end = min(kv_tokens, min(tok0 + kTok, q_tokens) + off);
-  // key range of this workgroup: whole rows, or one chunk of them
-  const unsigned kv_first = kSplit ? chunk * sp.chunk_keys : 0u;
-  const unsigned kv_stop = kSplit ? min(kv_end, kv_first + sp.chunk_keys) : kv_end;
-  if (kSplit && kv_first >= kv_end) return;   // past the tile's last key
+  // key range of this workgroup: whole rows, or one chunk of them (kSub = 2: of
+  // this half, which may be empty for the second)
+  const unsigned kv_wg = kSplit ? chunk * sp.chunk_keys : 0u;
+  if (kSplit && kv_wg >= kv_end) return;   // past the tile's last key
+  const unsigned sub_keys = sp.chunk_keys / kSub;
+  const unsigned kv_first = kv_wg + (kSub == 1 ? 0u : sub * sub_keys);
+  const unsigned kv_stop = kSplit ? min(kv_end, kv_first + sub_keys) : kv_end;
 
   // Q^T operand: step s covers dims s*16 + 8*lg .. +8 of this lane's row.
   bf16x8 qf[16];
@@ -208,14 +221,18 @@ __global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_pre
 
   const unsigned t_first = kv_first / kFmKv;
   const unsigned n_tiles = (kv_stop + kFmKv - 1) / kFmKv;
-  fetch(kv_first, t_first & 1);
-  for (unsigned t = t_first; t < n_tiles; ++t) {
+  // both halves pass as many barriers as the first has tiles (it has the most)
+  const unsigned t_end =
+      kSub == 1 ? n_tiles : t_first + (min(kv_end - kv_wg, sub_keys) + kFmKv - 1) / kFmKv;
+  if (kSub == 1 || t_first < n_tiles) fetch(kv_first, t_first & 1);
+  for (unsigned t = t_first; t < t_end; ++t) {
     const unsigned kv0 = t * kFmKv;
     const int stage = t & 1;
     __builtin_amdgcn_s_waitcnt(0);   // this wave's fetches of tile t landed
     __syncthreads();                 // ... and every wave's; tile t-1 consumed
     if (t + 1 < n_tiles) fetch(kv0 + kFmKv, stage ^ 1);
-    if (kv0 > wave_lim || !wave_live) continue;   // no row of ours sees a key of the tile
+    // no row of ours sees a key of the tile
+    if (kv0 > wave_lim || !wave_live || (kSub > 1 && t >= n_tiles)) continue;
     const char* kp = lds + stage * kFmStage + kbase;
     const char* vp = lds + stage * kFmStage + kKTile + vbase;
 
@@ -319,6 +336,35 @@ __global__ __launch_bounds__(64 * kFmWaves, kFmWaves == 8 ? 1 : 2) void fmha_pre
     __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
   }
   l += __shfl_xor(l, 32, 64);
+  if constexpr (kSub == 2) {
+    // the second half's (m, l, O) to LDS, lane by lane, and merged by the first
+    // (a half whose keys the row does not see has l = 0 and weighs nothing)
+    __syncthreads();   // every wave is done with the K/V rings
+    f32x4* xo = reinterpret_cast<f32x4*>(lds_all) + wave * 2048 + lane;
+    float2* xml = reinterpret_cast<float2*>(lds_all + kFmWaves * 32768) + wave * 64 + lane;
+    if (sub == 1) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i)
+        xo[i * 64] = f32x4{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1],
+                           o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+      *xml = float2{m, l};
+    }
+    __syncthreads();
+    if (sub == 1) return;
+    const float2 ml1 = *xml;
+    const float m_all = fmaxf(l == 0.f ? -INFINITY : m, ml1.y == 0.f ? -INFINITY : ml1.x);
+    const float w0 = l == 0.f ? 0.f : __builtin_amdgcn_exp2f(m - m_all);
+    const float w1 = ml1.y == 0.f ? 0.f : __builtin_amdgcn_exp2f(ml1.x - m_all);
+    m = m_all;
+    l = l * w0 + ml1.y * w1;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const f32x4 x = xo[i * 64];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[i >> 2][4 * (i & 3) + e] = o[i >> 2][4 * (i & 3) + e] * w0 + x[e] * w1;
+    }
+  }
   if constexpr (kSplit) {
     if (!row_valid) return;
     const size_t item = ((size_t)qtile * sp.n_chunks + chunk) * kHkv + kvh;
@@ -565,6 +611,21 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    32).  8 waves, whose tiles read K/V least often, from tokens x keys =
 //    1.4 M (256 over 8000: 54 us against 55; 64 over 64000: 86 against 98),
 //    4 waves below (93 over 8000: 34 us against 38), 2 waves below 0.1 M.
+//    Where 8 waves are chosen, pairs of 4-wave halves (kSub = 2) halve the
+//    partials' traffic (62 MB written and read back at 93 over 24000) but read
+//    each key twice as often, so they pay while a half has at most about 1250
+//    keys of at most 32768, from 6 tiles on, and where their tiles fill at least
+//    115 of the 128 workgroups per head.  Pairs / 8 waves of rows: 93 over 15000
+//    40.2 us / 46.3, 93 over 24000 50.9 / 56.6, 128 over 20000 55.0 / 63.3, 500 over
+//    2800 42.4 / 47.7, 670 over 2200 45.4 / 50.0; 150 over 30000, 1180 keys, 81.1 /
+//    86.5; but 93 over 50000 94.7 / 90.7, 500 over 60000, 7600 keys, 458 / 393, 64 over
+//    64000, 4 tiles, 101 / 87, 800 over 8000, 100 workgroups, 117 / 111.
+//    The items go to the XCDs in ranges where 2 to 12 tiles share chunks of
+//    at least 12000 keys in all (with / without, 93 over 24000 51.9 / 54.7, 150
+//    over 30000 82.0 / 87.1, 64 over 16000 35.6 / 39.2, 32 over 30000 35.7 / 39.0,
+//    64 over 64000 82.8 / 86.9; one tile: 16 over 8000 25.5 / 22.8; more tiles:
+//    256 over 8000 52.1 / 51.2, 1000 over 4000 91 / 85; short: 93 over 2000 26.1 /
+//    23.9).
 //    Up to 3072 rows two chunks still win (2500 over 4000: 219 us against
 //    299 unsplit; 3500: 339 against 325).
 //  * square prompts: later tiles hold more chunks, 2 tiles (n + 1) / 2 in
@@ -574,13 +635,14 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    200).  8-token tiles up to 360 tokens (256: 16 us against 17), 16-token
 //    tiles up to 960 (768: 29 us against 33; 1000: 37 against 36).
 struct SplitPlan {
-  unsigned waves, tiles, n_chunks, chunk_keys, items;   // items: (tile, chunk, KV head) partials
+  unsigned waves, sub, tiles, n_chunks, chunk_keys, ranges, items;   // items: (tile, chunk, KV head) partials
 };
 
 unsigned tile_tokens(unsigned waves) { return waves * kFmRowsPerWave / kGroup; }
 
 SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   SplitPlan p{};
+  p.sub = 1u;
   p.n_chunks = 1u;
   p.chunk_keys = kv_tokens;
   const bool square = kv_tokens - q_tokens < 256u;
@@ -590,6 +652,12 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
     p.waves = q_tokens <= 360u ? 2u : q_tokens <= 960u ? 4u : 8u;
   else
     p.waves = work <= 100000u ? 2u : work <= 1400000u ? 4u : 8u;
+  const unsigned pairs = (q_tokens + tile_tokens(4u) - 1) / tile_tokens(4u);
+  if (!square && p.waves == 8u && pairs >= 6u && pairs <= 42u && 128u / pairs * pairs >= 115u &&
+      kv_tokens <= 32768u && (size_t)pairs * kv_tokens <= 1250u * 256u) {
+    p.waves = 4u;
+    p.sub = 2u;
+  }
   p.tiles = (q_tokens + tile_tokens(p.waves) - 1) / tile_tokens(p.waves);
   unsigned n;
   if (square) {
@@ -598,17 +666,21 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
     n = std::min(128u / p.tiles, kv_tokens / 96u);
     n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
   }
-  const unsigned chunk = ((kv_tokens + n - 1) / n + kFmKv - 1) / kFmKv * kFmKv;
+  const unsigned quantum = kFmKv * p.sub;
+  const unsigned chunk = ((kv_tokens + n - 1) / n + quantum - 1) / quantum * quantum;
   n = (kv_tokens + chunk - 1) / chunk;   // after rounding up
   if (n < 2u) return p;
   p.n_chunks = n;
   p.chunk_keys = chunk;
+  p.ranges = !square && p.tiles > 1u && p.tiles <= 12u && kv_tokens >= 12000u;
   p.items = p.tiles * n * kHkv;          // at most kSplitItems
   return p;
 }
 
 size_t split_workspace_bytes(const SplitPlan& p) {
-  return p.n_chunks > 1 ? (size_t)p.items * (p.waves * kFmRowsPerWave) * (kD + 2) * sizeof(float) : 0;
+  // (pairs would do with half, but one size serves the neighbouring geometries)
+  return p.n_chunks > 1 ? (size_t)p.items * (p.waves * p.sub * kFmRowsPerWave) * (kD + 2) * sizeof(float)
+                        : 0;
 }
 
 // Whether the call may run with this workspace, and whether it then splits.
@@ -644,7 +716,11 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
           hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kFmLds);
       if (e != hipSuccess) g_fm_attr_status = e;
     }
-    const hipError_t e = hipFuncSetAttribute(
+    hipError_t e = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(fmha_prefill_kernel<4, true, false, 2>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kFmLds);
+    if (e != hipSuccess) g_fm_attr_status = e;
+    e = hipFuncSetAttribute(
         reinterpret_cast<const void*>(fmha_prefill_kernel<8, false, true>),
         hipFuncAttributeMaxDynamicSharedMemorySize, kFmLdsGated);
     if (e != hipSuccess) g_fm_attr_status = e;
@@ -660,11 +736,13 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
     sp.ml = sp.o + (size_t)plan.items * (plan.waves * kFmRowsPerWave) * kD;   // after the O partials
     sp.chunk_keys = plan.chunk_keys;
     sp.n_chunks = plan.n_chunks;
-    auto split = plan.waves == 8   ? fmha_prefill_kernel<8, true>
+    sp.ranges = plan.ranges;
+    auto split = plan.sub == 2     ? fmha_prefill_kernel<4, true, false, 2>
+                 : plan.waves == 8 ? fmha_prefill_kernel<8, true>
                  : plan.waves == 4 ? fmha_prefill_kernel<4, true>
                                    : fmha_prefill_kernel<2, true>;
     hipLaunchKernelGGL(split, dim3(8 * ((plan.tiles * plan.n_chunks + 3) / 4)),
-                       dim3(64 * plan.waves), kFmLds, stream, qb, kb, vb, out, q_tokens, kv_tokens,
+                       dim3(64 * plan.waves * plan.sub), kFmLds * plan.sub, stream, qb, kb, vb, out, q_tokens, kv_tokens,
                        plan.tiles, sp, ga);
     // groups of 32 threads per row: at most 4 chunks (one round trip) a group,
     // 8 past 64 chunks
@@ -690,7 +768,7 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
                        plan.n_chunks, ga);
     return static_cast<int>(hipGetLastError());
   }
-  const SplitArgs none{nullptr, nullptr, 0u, 1u};
+  const SplitArgs none{nullptr, nullptr, 0u, 1u, 0u};
   auto tiles = [&](unsigned waves) { return (q_tokens + tile_tokens(waves) - 1) / tile_tokens(waves); };
   auto grid = [&](unsigned waves) { return dim3(8 * ((tiles(waves) + 3) / 4)); };
   if (ga.out != nullptr) {   // gated: 256-row workgroups at every length

@@ -34,8 +34,8 @@ extern "C" {
  * [q_tokens,4096]; scale 1/16; top-left causal mask when
  * q_tokens == kv_tokens, bottom-right otherwise. */
 /* prepare (0 < tokens <= 262144) allocates, once per device, the provider's
- * 132 MiB split-K scratch: launches with fewer than 16 query tiles of 256
- * rows split each tile's key range over several workgroups plus a combine
+ * 132 MiB split-K scratch: launches of up to 4096 tokens (3072 over a prefix)
+ * split each tile's key range over several workgroups plus a combine
  * launch and use it (without it -- not prepared, or the allocation failed, in
  * which case prepare still returns 0 -- they run unsplit).  The first split
  * launch on a device claims the scratch for its stream: later launches on
