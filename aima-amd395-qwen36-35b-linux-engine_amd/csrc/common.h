@@ -75,16 +75,16 @@ constexpr float kLn2Lo = 4.888495152129525e-06f;    // (log2(e) - kLog2eHi) ln 2
 
 // x / (1 + e^-x) (SiLU as the reference's conv writes it) for a bf16 x,
 // from the hardware exp2 and reciprocal with the split log2(e) of
-// gate4_bf16_fast: within ~5 ulps of the exact form's value.  Sets `slow`
-// when that value could round to another bf16 than the exact one (within
-// 32 ulps of a rounding midpoint), or |x| > 60, or x is not finite.
-__device__ __forceinline__ float silu_fast(float x, bool& slow) {
+// gate4_bf16_fast.  For |x| <= 60 within 4 ulps of the true value (exp2, the
+// first-order factor, the sum, the reciprocal and the product at half to one
+// each), where the exact form is within 2.5: outside kSiluMid ulps of a
+// rounding midpoint both round to the same bf16.
+constexpr int kSiluMid = 8;
+constexpr unsigned kBf16Sixty = 0x4270u;   // the bits of 60
+__device__ __forceinline__ float silu_fast(float x) {
   const float th = __builtin_amdgcn_exp2f(x * -kLog2eHi);
   const float t = __builtin_fmaf(th, x * -kLn2Lo, th);
-  const float s = x * __builtin_amdgcn_rcpf(1.0f + t);
-  const int mid = (int)(__float_as_uint(s) & 0xffffu) - 0x8000;
-  slow = !(fabsf(x) <= 60.0f) || (mid >= -32 && mid <= 32);
-  return s;
+  return x * __builtin_amdgcn_rcpf(1.0f + t);
 }
 
 // gate_bf16 for four values, with the sigmoid from the hardware exp2 and

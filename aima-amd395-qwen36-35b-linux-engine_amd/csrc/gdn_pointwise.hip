@@ -66,10 +66,22 @@ __global__ __launch_bounds__(256) void gdn_conv1d_kernel(
   }
 }
 
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// Two values to bf16 (RNE) in one conversion, the first in the low half.
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
 // Vector form of gdn_conv1d_kernel (16-byte loads and stores, the same
 // conv arithmetic; SiLU through silu_fast with the exact form where it could
-// differ, so the same bits for every finite input): grid = (C/2048,
-// ceil(T/TPT)); thread = 8 consecutive channels, TPT consecutive tokens.
+// differ, so the same bits for every finite input).  Bound by VALU issue: with
+// the exact form within 32 ulps of a midpoint 40% of a wave's rows took it, within
+// 8 ulps 12% do, and the tests run on packed halves (the DeltaNet layer's
+// prefill, same box: 1000 tokens 151.9 -> 149.8 us, 8192 775.9 -> 772.1).
+// grid = (C/2048, ceil(T/TPT)); thread = 8 consecutive channels, TPT consecutive tokens.
 // Two load orders (MI355X, graph-replayed):
 //  * kUpfront: every row and the state requested unconditionally before
 //    the first use (the first block's three history rows read row 0 and
@@ -147,32 +159,42 @@ __global__ __launch_bounds__(256) void gdn_conv1d_vec_kernel(
   for (int j = 0; j < TPT; ++j) {
     const unsigned t = t0 + j;
     // SiLU from the hardware exp2 / rcp; the exact form only where the fast
-    // value could round to another bf16 (one branch per row of 8)
+    // value could round to another bf16, or |x| > 60 or x is not finite: both
+    // tested over the row's 8 values in packed 16-bit halves
     float cv[8], sv[8];
-    bool slow = false;
+    u16x2 near = {0xffff, 0xffff}, big = {0, 0};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float acc = mul_rn(val(j, e), w[e][0]);
-      acc = add_rn(acc, mul_rn(val(j + 1, e), w[e][1]));
-      acc = add_rn(acc, mul_rn(val(j + 2, e), w[e][2]));
-      acc = add_rn(acc, mul_rn(val(j + 3, e), w[e][3]));
-      cv[e] = bf2f(f2bf(acc));
-      bool sl;
-      sv[e] = silu_fast(cv[e], sl);
-      slow |= sl;
+    for (int e = 0; e < 8; e += 2) {
+      float acc[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        acc[u] = mul_rn(val(j, e + u), w[e + u][0]);
+        acc[u] = add_rn(acc[u], mul_rn(val(j + 1, e + u), w[e + u][1]));
+        acc[u] = add_rn(acc[u], mul_rn(val(j + 2, e + u), w[e + u][2]));
+        acc[u] = add_rn(acc[u], mul_rn(val(j + 3, e + u), w[e + u][3]));
+      }
+      const unsigned cb = pack_bf16(acc[0], acc[1]);
+      cv[e] = __uint_as_float(cb << 16);
+      cv[e + 1] = __uint_as_float(cb & 0xffff0000u);
+      sv[e] = silu_fast(cv[e]);
+      sv[e + 1] = silu_fast(cv[e + 1]);
+      const u16x2 low = __builtin_bit_cast(
+          u16x2, __builtin_amdgcn_perm(__float_as_uint(sv[e + 1]), __float_as_uint(sv[e]), 0x05040100u));
+      near = __builtin_elementwise_min(near, (u16x2)(low - (unsigned short)(0x8000 - kSiluMid)));
+      big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2, cb & 0x7fff7fffu));
     }
-    if (slow) {
+    if (min(near[0], near[1]) <= 2 * kSiluMid || max(big[0], big[1]) > kBf16Sixty) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        bool sl;
-        silu_fast(cv[e], sl);
-        if (sl) sv[e] = cv[e] / (1.0f + expf(-cv[e]));
+        const unsigned short d =
+            (unsigned short)((__float_as_uint(sv[e]) & 0xffffu) - (0x8000 - kSiluMid));
+        if (d <= 2 * kSiluMid || !(fabsf(cv[e]) <= 60.0f)) sv[e] = cv[e] / (1.0f + expf(-cv[e]));
       }
     }
-    bf16x8 o;
+    u32x4 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = f2bf(sv[e]);
-    if (t < tokens) *reinterpret_cast<bf16x8*>(out + (size_t)t * kGdnConvDim + c0) = o;
+    for (int e = 0; e < 8; e += 2) o[e / 2] = pack_bf16(sv[e], sv[e + 1]);
+    if (t < tokens) *reinterpret_cast<u32x4*>(out + (size_t)t * kGdnConvDim + c0) = o;
   }
   // The first token block owns the state update (state_in may alias
   // state_out: this thread read its state above).
