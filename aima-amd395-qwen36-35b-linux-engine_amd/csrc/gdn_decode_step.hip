@@ -35,11 +35,6 @@ namespace {
 #endif
 constexpr int kDsThreads = DS_THREADS;
 constexpr int kDsWaves = kDsThreads / 64;
-// The heads fill 32 of the 256 CUs: where the caller names what the next launch
-// streams (out_proj, 16.8 MB), as many workgroups as there are CUs left read it
-// into L2 beside them, in the 64 KiB pieces of the GEMV's workgroups (MI355X, six
-// layers with projections: 128.7 us without, 125.5 with).
-constexpr unsigned kDsWarmGroups = 224;
 constexpr int kDsRowsPerThread = kGdnDk / (kDsThreads / 32);   // row groups of 32 threads
 
 __device__ __forceinline__ float ds_mul(float a, float b) { return __fmul_rn(a, b); }
@@ -53,11 +48,7 @@ __global__ __launch_bounds__(kDsThreads) void gdn_decode_step_kernel(
     const float* __restrict__ a_log, const float* __restrict__ dt_bias,
     const bf16* __restrict__ z, unsigned z_row_stride,
     const bf16* __restrict__ norm_w, const float* state_in, float* state_out,
-    bf16* __restrict__ out, unsigned tokens, const void* next, unsigned next_bytes) {
-  if (blockIdx.x >= kGdnHv) {
-    warm_l2<kWarmPiece, kDsThreads>(next, next_bytes, blockIdx.x - kGdnHv, kDsWarmGroups);
-    return;
-  }
+    bf16* __restrict__ out, unsigned tokens) {
   __shared__ float ych[2][3 * kGdnDk];              // [parity][q | k | v] conv outputs
   __shared__ float gb[2][2];                        // [parity][g, beta]
   __shared__ f32x4 red[2][kDsWaves][2][32];         // [parity][wave][kv | sq][col quad]
@@ -237,13 +228,13 @@ static bool ranges_overlap(const void* p, const void* q, size_t n) {
   return a < b + n && b < a + n;
 }
 
-Q36_EXPORT int qwen36_gdn_decode_step_next(
+Q36_EXPORT int qwen36_gdn_decode_step(
     const void* mixed_qkv, unsigned x_row_stride, const void* conv_weight,
     const void* conv_state_in, void* conv_state_out, const void* a,
     const void* b, unsigned ab_row_stride, const void* a_log,
     const void* dt_bias, const void* z, unsigned z_row_stride,
     const void* norm_weight, const void* state_in, void* state_out, void* out,
-    unsigned tokens, const void* next_weight, size_t next_bytes, void* stream) {
+    unsigned tokens, void* stream) {
   const size_t conv_bytes = (size_t)kGdnConvDim * 3 * sizeof(bf16);
   if (mixed_qkv == nullptr || conv_weight == nullptr || conv_state_in == nullptr ||
       conv_state_out == nullptr || a == nullptr || b == nullptr || a_log == nullptr ||
@@ -254,12 +245,9 @@ Q36_EXPORT int qwen36_gdn_decode_step_next(
       (z_row_stride % 4) != 0 || ranges_overlap(conv_state_in, conv_state_out, conv_bytes) ||
       (reinterpret_cast<uintptr_t>(z) % 8) != 0 || (reinterpret_cast<uintptr_t>(out) % 8) != 0 ||
       (reinterpret_cast<uintptr_t>(state_in) % 16) != 0 ||
-      (reinterpret_cast<uintptr_t>(state_out) % 16) != 0 ||
-      (next_weight == nullptr) != (next_bytes == 0) || next_bytes > kWarmMax ||
-      (reinterpret_cast<uintptr_t>(next_weight) % 16) != 0)
+      (reinterpret_cast<uintptr_t>(state_out) % 16) != 0)
     return Q36_EINVAL;
-  hipLaunchKernelGGL(gdn_decode_step_kernel,
-                     dim3(kGdnHv + (next_weight != nullptr ? kDsWarmGroups : 0)), dim3(kDsThreads), 0,
+  hipLaunchKernelGGL(gdn_decode_step_kernel, dim3(kGdnHv), dim3(kDsThreads), 0,
                      static_cast<hipStream_t>(stream),
                      static_cast<const bf16*>(mixed_qkv), x_row_stride,
                      static_cast<const bf16*>(conv_weight),
@@ -270,19 +258,6 @@ Q36_EXPORT int qwen36_gdn_decode_step_next(
                      static_cast<const bf16*>(z), z_row_stride,
                      static_cast<const bf16*>(norm_weight),
                      static_cast<const float*>(state_in), static_cast<float*>(state_out),
-                     static_cast<bf16*>(out), tokens, next_weight, (unsigned)next_bytes);
+                     static_cast<bf16*>(out), tokens);
   return static_cast<int>(hipGetLastError());
-}
-
-Q36_EXPORT int qwen36_gdn_decode_step(
-    const void* mixed_qkv, unsigned x_row_stride, const void* conv_weight,
-    const void* conv_state_in, void* conv_state_out, const void* a,
-    const void* b, unsigned ab_row_stride, const void* a_log,
-    const void* dt_bias, const void* z, unsigned z_row_stride,
-    const void* norm_weight, const void* state_in, void* state_out, void* out,
-    unsigned tokens, void* stream) {
-  return qwen36_gdn_decode_step_next(mixed_qkv, x_row_stride, conv_weight, conv_state_in,
-                                     conv_state_out, a, b, ab_row_stride, a_log, dt_bias, z,
-                                     z_row_stride, norm_weight, state_in, state_out, out, tokens,
-                                     nullptr, 0, stream);
 }

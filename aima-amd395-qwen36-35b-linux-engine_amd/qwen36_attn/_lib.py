@@ -93,9 +93,6 @@ SIGNATURES: dict[str, tuple] = {
     "qwen36_prefix_cache_destroy": (_i32, [_vp]),
     "qwen36_gdn_decode_step": (_i32, [_vp, _u32, _vp, _vp, _vp, _vp, _vp, _u32, _vp,
                                       _vp, _vp, _u32, _vp, _vp, _vp, _vp, _u32, _vp]),
-    "qwen36_gdn_decode_step_next": (_i32, [_vp, _u32, _vp, _vp, _vp, _vp, _vp, _u32, _vp,
-                                           _vp, _vp, _u32, _vp, _vp, _vp, _vp, _u32, _vp, _sz,
-                                           _vp]),
 }
 
 _LIB = None

@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._tensors import ptr, read_ahead, require, scratch, stream_handle
+from ._tensors import ptr, require, scratch, stream_handle
 
 HK, HV, DK, DV = 16, 32, 128, 128
 KEY_DIM, VALUE_DIM = HK * DK, HV * DV
@@ -210,17 +210,14 @@ def gdn_decode_step(mixed_qkv: torch.Tensor, conv_state: torch.Tensor,
                     a: torch.Tensor, b: torch.Tensor, a_log: torch.Tensor,
                     dt_bias: torch.Tensor, z: torch.Tensor, norm_weight: torch.Tensor,
                     ssm_state: torch.Tensor, final_state: torch.Tensor | None = None,
-                    out: torch.Tensor | None = None,
-                    next_weight: torch.Tensor | None = None) -> torch.Tensor:
+                    out: torch.Tensor | None = None) -> torch.Tensor:
     """One fused launch for the decode part of ``linear_attention`` between
     the input projections and out_proj (fle:6378-6544, mode "decode"): conv
     + SiLU, gating, l2norm, recurrent delta rule and gated RMSNorm for the
     T rows of ``mixed_qkv``.  ``new_conv_state`` receives the conv state and
     must be a different buffer from ``conv_state``; ``final_state`` (default:
-    ``ssm_state`` itself) receives the fp32 recurrent state.  ``next_weight``
-    (out_proj): what the next launch streams, read into L2 by CUs that the
-    heads leave idle; the results are the same.  Returns the gated output
-    [T, 4096] bf16."""
+    ``ssm_state`` itself) receives the fp32 recurrent state.  Returns the
+    gated output [T, 4096] bf16."""
     t = mixed_qkv.shape[0]
     require(mixed_qkv, "mixed_qkv", torch.bfloat16, contiguous=False)
     if mixed_qkv.shape[1] != CONV_DIM or mixed_qkv.stride(1) != 1:
@@ -249,10 +246,10 @@ def gdn_decode_step(mixed_qkv: torch.Tensor, conv_state: torch.Tensor,
     dt_bias = dt_bias.float().contiguous()
     if out is None:
         out = torch.empty(t, VALUE_DIM, dtype=torch.bfloat16, device=mixed_qkv.device)
-    _lib.call("qwen36_gdn_decode_step_next", ptr(mixed_qkv), mixed_qkv.stride(0), ptr(conv_weight),
+    _lib.call("qwen36_gdn_decode_step", ptr(mixed_qkv), mixed_qkv.stride(0), ptr(conv_weight),
               ptr(conv_state), ptr(new_conv_state), ptr(a), ptr(b), a.stride(0), ptr(a_log),
               ptr(dt_bias), ptr(z), z.stride(0), ptr(norm_weight), ptr(ssm), ptr(final_state),
-              ptr(out), t, *read_ahead(next_weight, out.device), stream_handle(out.device))
+              ptr(out), t, stream_handle(out.device))
     return out
 
 
@@ -301,8 +298,7 @@ class LinearAttentionLayer:
             if self.conv_spare is None:
                 self.conv_spare = torch.empty_like(self.conv_state)
             gated = gdn_decode_step(mixed, self.conv_state, self.conv_spare, w["conv1d"], a, b,
-                                    w["A_log"], w["dt_bias"], z, w["norm"], self.ssm_state,
-                                    next_weight=w["out_proj"])
+                                    w["A_log"], w["dt_bias"], z, w["norm"], self.ssm_state)
             self.conv_state, self.conv_spare = self.conv_spare, self.conv_state
             return gemv(w["out_proj"], gated)
         from .prefill_gemm import linear

@@ -210,8 +210,7 @@ def linear_attention(inp: torch.Tensor, layer_index: int, weights: dict) -> torc
     if st.mode == "decode":
         gated = gd.gdn_decode_step(mixed, conv_in, conv_out, cw, a, b, w["linear_A_log"],
                                    w["linear_dt_bias"], z, w["linear_norm"], ssm_in,
-                                   final_state=ssm_out,
-                                   next_weight=w["linear_out_proj"] if t == 1 else None)
+                                   final_state=ssm_out)
         return gemv(w["linear_out_proj"], gated) if t == 1 else pg.linear(gated, w["linear_out_proj"])
     conv, _ = gd.causal_conv1d(mixed, conv_in, cw, new_state=conv_out)
     q = conv[:, :gd.KEY_DIM].view(t, gd.HK, gd.DK)

@@ -325,18 +325,6 @@ int qwen36_gdn_decode_step(const void* mixed_qkv, unsigned x_row_stride,
                            const void* state_in, void* state_out, void* out,
                            unsigned tokens, void* stream);
 
-/* qwen36_gdn_decode_step_next: the same, told what the next launch streams
- * (out_proj; see qwen36_decode_step_next). */
-int qwen36_gdn_decode_step_next(const void* mixed_qkv, unsigned x_row_stride,
-                                const void* conv_weight, const void* conv_state_in,
-                                void* conv_state_out, const void* a, const void* b,
-                                unsigned ab_row_stride, const void* a_log,
-                                const void* dt_bias, const void* z,
-                                unsigned z_row_stride, const void* norm_weight,
-                                const void* state_in, void* state_out, void* out,
-                                unsigned tokens, const void* next_weight,
-                                size_t next_bytes, void* stream);
-
 /* ---- prefill projections ---------------------------------------------------
  * qwen36_prefill_gemm_bf16: y[m, n] = x[m, k] W[n, k]^T for a prompt of m
  * tokens, bf16 in and out with fp32 accumulation (one rounding); replaces

@@ -1,4 +1,4 @@
-"""Decode steps told what the next launch streams: the workgroups that read it
+"""The attention decode step told what the next launch streams: the workgroups that read it
 ahead change nothing, whatever its size (a ragged last piece, one 16-byte row,
 more pieces than workgroups) and whether or not the split leaves room for them
 (up to 128 split workgroups), and the hint never refuses a call."""
@@ -6,7 +6,6 @@ import pytest
 import torch
 
 from qwen36_attn import synthetic as syn
-from tests.test_gdn_decode_step_gpu import _step_inputs
 
 BF16 = torch.bfloat16
 ELEMENTS = [8, 32768 + 24, 2048 * 4096, 16 << 20]
@@ -42,34 +41,11 @@ def test_attention_step_with_next_weight(gpu, rows, split, elements):
     assert torch.equal(w, w0)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("elements", ELEMENTS)
-@pytest.mark.parametrize("tokens", [1, 3])
-def test_gdn_step_with_next_weight(gpu, tokens, elements):
-    from qwen36_attn.gated_deltanet import gdn_decode_step
-    mixed, conv_w, conv, a, b, a_log, dt, z, nw, ssm = (
-        x.to(gpu) for x in _step_inputs(tokens, 7, 1.0))
-    w = syn.randn((elements,), syn.gen(2)).to(gpu)
-    w0 = w.clone()
-    print(f"gdn step tokens={tokens} next={elements}", flush=True)
-    outs = []
-    for nxt in (w, None):
-        new_conv, state = torch.empty_like(conv), torch.empty_like(ssm)
-        out = gdn_decode_step(mixed, conv, new_conv, conv_w, a, b, a_log, dt, z, nw, ssm,
-                              final_state=state, next_weight=nxt)
-        outs.append((out, new_conv, state))
-    torch.cuda.synchronize()
-    assert all(torch.equal(x, y) for x, y in zip(*outs))
-    assert torch.equal(w, w0)
-
-
 def test_next_weight_refusals():
     """C entries: bytes without an address, an address without bytes, more than
     the L2s hold, an address off 16 bytes."""
     from qwen36_attn import _lib
-    L = _lib.load(("qwen36_decode_step_next", "qwen36_gdn_decode_step_next"))
+    L = _lib.load(("qwen36_decode_step_next",))
     for nxt in ((None, 16), (32, 0), (32, (32 << 20) + 1), (40, 16)):
         assert L.qwen36_decode_step_next(16, 16, 16, 16, 16, 16, 16, 0, 1, 1, 16, 16, 1 << 30, 0,
                                          *nxt, None) == 1
-        assert L.qwen36_gdn_decode_step_next(16, 8192, 32, 4096, 1 << 20, 48, 64, 32, 80, 96, 128,
-                                             4096, 160, 256, 256, 512, 1, *nxt, None) == 1
