@@ -446,11 +446,11 @@ __global__ __launch_bounds__(64 * kFmWaves * kSub, kFmWaves * kSub == 8 ? 1 : 2)
 // Split-K combine: kG groups of 32 threads (8 dims each) merge the live
 // chunks' partials of one (token, head) row, group g chunks g, g + kG, ...:
 // M = max m_c, L = sum l_c 2^(m_c - M), O = sum O_c 2^(m_c - M) / L (chunks
-// where the row saw no key have l = 0 and weigh nothing), then the groups
-// through LDS, in group order.  block = 512 = 16 / kG rows of 32 kG threads.
+// where the row saw no key have l = 0 and weigh nothing; a NaN l, from a
+// non-finite key or query, is kept and makes the row NaN, as without a split),
+// then the groups through LDS, in group order.  block = 512 = 16 / kG rows of 32 kG threads.
 // A group's (m, l) pairs, its first four chunks' O partials and the gate
 // are requested together (indices clamped to the live range, so every load
-// is unconditional and in bounds): one memory round trip for up to four
 // is unconditional and in bounds): one memory round trip for up to four
 // chunks a group, so the launch picks kG for at most four.  The reads bound
 // it: 42 chunks of 93 tokens, 62 MB, 12.9 us (with 8 groups of up to 16
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
   float M = -INFINITY;
 #pragma unroll
   for (int c = 0; c < kMaxC; ++c)
-    if (g + kG * c < live && ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
+    if (g + kG * c < live && ml[c].y != 0.f) M = fmaxf(M, ml[c].x);
   float L = 0.f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int c0 = 0; c0 < kMaxC; c0 += 4) {
@@ -508,7 +508,7 @@ __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float2 m_l = ml[c0 + j];
-      if (g + kG * (c0 + j) < live && m_l.y > 0.f) {
+      if (g + kG * (c0 + j) < live && m_l.y != 0.f) {
         const float w = __builtin_amdgcn_exp2f(m_l.x - M);
         L += w * m_l.y;
 #pragma unroll
@@ -526,17 +526,17 @@ __global__ __launch_bounds__(512) void fmha_split_combine_kernel(
     if ((threadIdx.x & 31) == 0) part_ml[threadIdx.x >> 5] = float2{M, L};
     __syncthreads();
     if (g != 0) return;
-    float m_all = M;   // key 0's chunk is live: some group has L > 0
+    float m_all = M;   // key 0's chunk is live: some group has L != 0
 #pragma unroll
     for (int j = 1; j < kG; ++j) m_all = fmaxf(m_all, part_ml[(threadIdx.x >> 5) + j].x);
-    const float w0 = L > 0.f ? __builtin_amdgcn_exp2f(M - m_all) : 0.f;
+    const float w0 = L != 0.f ? __builtin_amdgcn_exp2f(M - m_all) : 0.f;
     L *= w0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] *= w0;
 #pragma unroll
     for (int j = 1; j < kG; ++j) {
       const float2 m_l = part_ml[(threadIdx.x >> 5) + j];
-      const float w = m_l.y > 0.f ? __builtin_amdgcn_exp2f(m_l.x - m_all) : 0.f;
+      const float w = m_l.y != 0.f ? __builtin_amdgcn_exp2f(m_l.x - m_all) : 0.f;
       L += w * m_l.y;
       const f32x4* src = reinterpret_cast<const f32x4*>(part[threadIdx.x + 32 * j]);
       const f32x4 a = src[0], b = src[1];
