@@ -125,6 +125,22 @@ def decode_step(q_gate: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return out
 
 
+# Up to this many query tokens a split needs its workspace (the C entries refuse
+# the call without) and the calls of a device share one buffer.  Longer ones can
+# run unsplit, so they take memory of their own: they need no eager call before a
+# capture and may run on several streams at once.
+_SHARED_SPLIT_TOKENS = 2560
+
+
+def _split_workspace(t: int, s: int, device: torch.device) -> torch.Tensor | None:
+    nb = _lib.load(("qwen36_fmha_prefill_workspace_bytes",)).qwen36_fmha_prefill_workspace_bytes(t, s)
+    if not nb:
+        return None
+    if t > _SHARED_SPLIT_TOKENS:
+        return torch.empty(nb, dtype=torch.uint8, device=device)
+    return scratch("fmha_split", nb, device)
+
+
 def fmha_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                  out: torch.Tensor | None = None) -> torch.Tensor:
     """Causal GQA flash attention, the computation of the provider ABI
@@ -149,9 +165,8 @@ def fmha_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if out is None:
         out = torch.empty(t, Q_DIM, dtype=torch.float32, device=q.device)
     require(out, "out", torch.float32, shape=(t, Q_DIM))
-    lib = _lib.load(("qwen36_fmha_prefill",))
-    nb = lib.qwen36_fmha_prefill_workspace_bytes(t, s)
-    ws = scratch("fmha_split", nb, q.device) if nb else None
+    _lib.load(("qwen36_fmha_prefill",))
+    ws = _split_workspace(t, s, q.device)
     _lib.call("qwen36_fmha_prefill", ptr(q), ptr(k), ptr(v), ptr(out), t, s, ptr(ws),
               ws.numel() if ws is not None else 0, stream_handle(q.device))
     return out
@@ -184,9 +199,8 @@ def fmha_prefill_gated(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if out is None:
         out = torch.empty(t, Q_DIM, dtype=torch.bfloat16, device=q.device)
     require(out, "out", torch.bfloat16, shape=(t, Q_DIM))
-    lib = _lib.load(("qwen36_fmha_prefill_gated",))
-    nb = lib.qwen36_fmha_prefill_workspace_bytes(t, s)
-    ws = scratch("fmha_split", nb, q.device) if nb else None
+    _lib.load(("qwen36_fmha_prefill_gated",))
+    ws = _split_workspace(t, s, q.device)
     _lib.call("qwen36_fmha_prefill_gated", ptr(q), ptr(k), ptr(v), ptr(q_gate), q_gate.stride(0),
               ptr(out), t, s, ptr(ws), ws.numel() if ws is not None else 0,
               stream_handle(q.device))
