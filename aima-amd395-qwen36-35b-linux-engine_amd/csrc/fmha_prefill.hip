@@ -677,10 +677,17 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   return p;
 }
 
+// One size serves every split of up to 2560 tokens, so a buffer that one of them
+// sized is enough for the others, whatever their length and prefix (a shared buffer
+// does not grow during a capture).  The most is 66 tiles of 32 tokens in 3 chunks
+// for 2 KV heads: square prompts make at most 42 x 4, 66 x 3 or 80 x 2 (tile, chunk)
+// pairs, rows over a prefix at most 128 or 80 x 2.  Longer prompts take at least as much.
+constexpr size_t kSplitSharedBytes = 66 * 3 * kHkv * kSplitItemBytes;
+
 size_t split_workspace_bytes(const SplitPlan& p) {
-  // (pairs would do with half, but one size serves the neighbouring geometries)
-  return p.n_chunks > 1 ? (size_t)p.items * (p.waves * p.sub * kFmRowsPerWave) * (kD + 2) * sizeof(float)
-                        : 0;
+  if (p.n_chunks < 2) return 0;
+  return std::max(kSplitSharedBytes,
+                  (size_t)p.items * (p.waves * p.sub * kFmRowsPerWave) * (kD + 2) * sizeof(float));
 }
 
 // Whether the call may run with this workspace, and whether it then splits.

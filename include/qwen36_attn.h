@@ -57,9 +57,10 @@ int qrt_ck_fmha_release(void);
  * prompts split on any stream: workspace of at least
  * qwen36_fmha_prefill_workspace_bytes(query_tokens, kv_tokens) bytes (0 =
  * this geometry runs unsplit and workspace may be NULL; also 0 for invalid
- * geometry, which the launch rejects).  From 2561 query tokens on the
- * workspace is optional: without enough of it the launch runs unsplit.  Calls
- * that overlap on one workspace race. */
+ * geometry, which the launch rejects).  Up to 2560 query tokens the size is
+ * one for all geometries that split, so one buffer serves them.  From 2561
+ * query tokens on the workspace is optional: without enough of it the launch
+ * runs unsplit.  Calls that overlap on one workspace race. */
 size_t qwen36_fmha_prefill_workspace_bytes(unsigned query_tokens, unsigned kv_tokens);
 int qwen36_fmha_prefill(const void* q, const void* k, const void* v, float* out,
                         unsigned query_tokens, unsigned kv_tokens, void* workspace,
