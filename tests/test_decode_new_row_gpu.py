@@ -3,11 +3,20 @@ the edges of a block, of the waves and of the rounds, with stale cache rows."""
 import pytest
 import torch
 
-from oracle import attention_oracle as O
+from oracle.attention_bounds import Row
 
 pytestmark = pytest.mark.gpu
 
-TOL = 2e-2   # bf16 output (P and the output rounded to bf16)
+
+def _check(out, q, k, v, lost):
+    """The output against 64 bits: P rounded to bf16 (Row), then the output (2^-8 of it at
+    most).  Each of ``lost`` (a range of keys) left out would be seen."""
+    row = Row(q, k, v)
+    tol = row.tol + 2.0 ** -8 * row.ref.abs()
+    assert ((out.cpu().double().view(4096) - row.ref).abs() <= tol).all()
+    for keys in lost:
+        if row.s > keys.stop - keys.start:
+            assert ((row.without(keys) - row.ref).abs() > 2 * tol).any(), keys
 
 
 @pytest.mark.parametrize("position,cache_end", [
@@ -18,6 +27,7 @@ def test_new_row_over_stale_cache(gpu, position, cache_end):
     g = torch.Generator().manual_seed(position + cache_end)
     q = torch.randn(16, 256, generator=g).to(torch.bfloat16)
     k, v = (torch.randn(cache_end, 2, 256, generator=g).to(torch.bfloat16) for _ in range(2))
+    v[position] *= 16             # a row that is left out shows
     kn, vn = k[position].clone(), v[position].clone()
     kd, vd = k.to(gpu), v.to(gpu)
     kd[position] = float("nan")   # whatever the row held is neither read nor used
@@ -25,8 +35,7 @@ def test_new_row_over_stale_cache(gpu, position, cache_end):
     out = decode_gqa(q.to(gpu), kd, vd, position, cache_end, kn.to(gpu), vn.to(gpu))
     torch.cuda.synchronize()
     assert torch.equal(kd[position].cpu(), kn) and torch.equal(vd[position].cpu(), vn)
-    ref = O.decode_attention_f32(q, k, v, cache_end)
-    assert (out.cpu().float() - ref.reshape(1, 4096).float()).abs().max().item() <= TOL
+    _check(out, q, k, v, [slice(position, position + 1)])
 
 
 @pytest.mark.parametrize("cache_end,split_tokens", [
@@ -40,5 +49,10 @@ def test_combine_forms(gpu, cache_end, split_tokens):
     k, v = (torch.randn(cache_end, 2, 256, generator=g).to(torch.bfloat16) for _ in range(2))
     out = decode_gqa(q.to(gpu), k.to(gpu), v.to(gpu), cache_end - 1, cache_end,
                      split_tokens=split_tokens)
-    ref = O.decode_attention_f32(q, k, v, cache_end)
-    assert (out.cpu().float() - ref.reshape(1, 4096).float()).abs().max().item() <= TOL
+    # blocks of 32 keys are dealt to the splits in turn
+    nsplit = (cache_end + split_tokens - 1) // split_tokens
+    blocks = torch.arange(cache_end) // 32
+    _check(out, q, k, v, [])
+    row = Row(q, k, v)
+    for split in {0, 1, nsplit // 2, nsplit - 16, nsplit - 1} & set(range(nsplit)):
+        assert row.sees(torch.nonzero(blocks % nsplit == split).flatten()), split

@@ -3,7 +3,7 @@ and of the coarse rule, and workspaces."""
 import pytest
 import torch
 
-from oracle import attention_oracle as O
+from oracle.attention_bounds import Row
 
 
 def test_workspace_serves_every_shorter_cache():
@@ -26,11 +26,13 @@ def test_default_split_matches_oracle(gpu, cache_end):
     qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
     print(f"decode splits cache_end={cache_end}", flush=True)
     out = decode_gqa(qd, kd, vd, cache_end - 1, cache_end)
-    ref = O.decode_attention_f32(q, k, v, cache_end).reshape(1, 4096)
-    # P enters the PV products as bf16 (at most 2^-9 of the largest value), the
-    # output is rounded to bf16
-    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -9 * v.float().abs().max() + 1e-4
-    assert ((out.cpu().float() - ref).abs() <= bound).all()
+    # P enters the PV products as bf16, the output is rounded to bf16
+    row = Row(q, k, v)
+    bound = 2.0 ** -8 * row.ref.abs() + row.tol
+    assert ((out.cpu().double().view(4096) - row.ref).abs() <= bound).all()
+    if cache_end > 32:   # one block of the least split left out shows
+        for block in (slice(0, 32), slice((cache_end - 1) // 32 * 32, cache_end)):
+            assert ((row.without(block) - row.ref).abs() > 2 * bound).any(), block
     # a workspace with room for 128-token splits only is still accepted, and
     # gives what that split size gives
     lib = _lib.load(("qwen36_decode_gqa",))

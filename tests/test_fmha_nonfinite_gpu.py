@@ -7,7 +7,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-TOL = 5e-3   # P rounded to bf16 (2^-9 relative) in sums that stay below |v| ~ 5
+TOL = 5 * 2.0 ** -8 + 1e-4   # P rounded to bf16 (2^-8 of each at most), |v| below 5
 
 
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
@@ -35,7 +35,7 @@ def test_nonfinite_key(gpu, t, s, key, bad):
     # wave with rows that see it, whose sums make the wave take new maxima, so
     # their P is rounded anew
     assert torch.equal(got[:, :8], clean[:, :8])
-    assert ((got[~sees] - clean[~sees]).abs() <= TOL).all()
+    assert ((got[~sees] - clean[~sees]).abs() <= 2 * TOL).all()
     got, qk = got[sees][:, 8:], q[sees][:, 8:, 7].float()
     if math.isnan(bad):
         assert got.isnan().all()
