@@ -1,7 +1,8 @@
 """The attention decode step told what the next launch streams: the workgroups that read it
 ahead change nothing, whatever its size (a ragged last piece, one 16-byte row,
-more pieces than workgroups) and whether or not the split leaves room for them
-(up to 128 split workgroups), and the hint never refuses a call."""
+more pieces than workgroups), with one split workgroup per KV head, with the most
+(128 beside 128 readers, 4096 rows) and where nothing is read ahead any more (4097
+rows), and the hint never refuses a call."""
 import pytest
 import torch
 
@@ -23,7 +24,8 @@ def test_read_ahead_hint_is_optional():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("elements", ELEMENTS)
-@pytest.mark.parametrize("rows,split", [(1, 0), (2051, 0), (8192, 0), (8193, 0), (8192, 128)])
+@pytest.mark.parametrize("rows,split", [(1, 0), (97, 0), (2051, 0), (2051, 1024), (4096, 0), (4096, 128),
+                                        (4097, 0), (8193, 0)])
 def test_attention_step_with_next_weight(gpu, rows, split, elements):
     from qwen36_attn.full_attention import decode_step
     g = syn.gen(rows)
