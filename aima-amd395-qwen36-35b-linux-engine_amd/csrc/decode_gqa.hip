@@ -60,9 +60,14 @@ constexpr unsigned kTargetSplits = 128;
 // launch (each workgroup's LDS fills a CU): where the caller names what the
 // launch after the combine streams (o_proj, 16.8 MB), as many more workgroups
 // read it into L2 meanwhile.  From 4097 cached tokens on they only compete with
-// the K and V stream.  MI355X, us a layer with projections, without / with: 400
-// rows 23.6 / 22.7, 2051 24.1 / 23.6, 4096 24.9 / 24.5, 6000 25.5 / 25.9, 8192
-// 26.5 / 27.1.
+// the K and V stream (6000 rows 25.5 / 25.9, 8192 26.5 / 27.1).  MI355X, us a layer
+// with projections, without / with, 12 layers of distinct weights (650 MB, which no
+// cache holds): 130 rows 23.3 / 22.5, 400 23.5 / 22.7, 1000 23.7 / 23.0, 2051 24.0 /
+// 23.6, 4096 24.8 / 24.6; each beside three DeltaNet layers (790 MB) 86.4 / 85.0 at
+// 130, 87.2 / 86.2 at 2051, 88.0 / 87.3 at 4096.  Weights that the Infinity Cache
+// holds gain less or lose (4 layers, two boxes: 2051 24.1 / 23.6 and 24.1 / 24.3,
+// 4096 25.0 / 24.4 and 24.9 / 25.5; 2 layers 24.6 / 25.2 and 25.5); a whole model's
+// are never there.
 constexpr unsigned kDecWarmGroups = 128, kDecWarmEnd = 4096;
 
 // RoPE inverse frequencies for the fused decode step (this translation
