@@ -614,12 +614,15 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    Where 8 waves are chosen, pairs of 4-wave halves (kSub = 2) halve the
 //    partials' traffic (62 MB written and read back at 93 over 24000) but read
 //    each key twice as often, so they pay while a half has at most about 1250
-//    keys of at most 32768, from 6 tiles on, and where their tiles fill at least
-//    115 of the 128 workgroups per head.  Pairs / 8 waves of rows: 93 over 15000
-//    40.2 us / 46.3, 93 over 24000 50.9 / 56.6, 128 over 20000 55.0 / 63.3, 500 over
-//    2800 42.4 / 47.7, 670 over 2200 45.4 / 50.0; 150 over 30000, 1180 keys, 81.1 /
-//    86.5; but 93 over 50000 94.7 / 90.7, 500 over 60000, 7600 keys, 458 / 393, 64 over
-//    64000, 4 tiles, 101 / 87, 800 over 8000, 100 workgroups, 117 / 111.
+//    keys of at most 32768 and where their tiles fill at least 115 of the 128
+//    workgroups per head.  Pairs / 8 waves of rows:
+//      pay: 93 over 15000 40.2 us / 46.3, over 24000 50.9 / 56.6; 128 over 20000
+//        55.0 / 63.3; 500 over 2800 42.4 / 47.7; 150 over 30000 (1180 keys) 81.1 / 86.5
+//      keys: 93 over 50000 94.7 / 90.7; 500 over 60000 (7600 keys) 458 / 393
+//      workgroups: 800 over 8000 (100 of 128) 117 / 111
+//    They are taken from 6 tiles on, which is no measured limit: 5 tiles (65 to
+//    80 tokens) would gain too (65 over 18000 41.3 / 41.2, 70 over 20000 42.4 /
+//    46.0, 75 over 24000 46.3 / 50.6, 80 over 28000 53.1 / 56.6), 4 are not measured.
 //    The items go to the XCDs in ranges where 2 to 12 tiles share chunks of
 //    at least 12000 keys in all (with / without, 93 over 24000 51.9 / 54.7, 150
 //    over 30000 82.0 / 87.1, 64 over 16000 35.6 / 39.2, 32 over 30000 35.7 / 39.0,

@@ -250,8 +250,9 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
 // padding; the shared expert is group E with slots 8T + t;
 // group g occupies rows [row_off[g], row_off[g] + roundup32(n_g)).  meta
 // (int4) [0] = {tiles}, [1 + i] = {group, first row, rows, tiles of the
-// group} for tile i; a group's rows are dealt evenly to its tiles, so that
-// 130 rows make two tiles of 96 and 34 and not 128 and 2.
+// group} for tile i; a group's rows are dealt evenly to its tiles in whole
+// blocks of 32: 300 rows make two 256-row tiles of 160 and 140, not 256 and 44
+// (64-row tiles leave nothing to deal: full tiles and a rest).
 // The 8T ids are cut into chunks of kAlignChunk: hist[g][chunk] counts, the
 // scan turns them into each chunk's first row per group, the scatter places
 // the chunk's slots.  Order inside a
