@@ -18,8 +18,8 @@
 //    rows a tile spans 32 tokens instead of 256, so a short turn fills its
 //    tiles (93 tokens: 3 tiles per KV head, all but 24 of 768 rows live, where
 //    256-token tiles of 8 heads left 163 of every 256 rows dead) and only a
-//    tile's last 32 keys are masked.  Fewer than 32 tokens use 4- or 2-wave
-//    workgroups (16 or 8 tokens).
+//    tile's last 32 keys are masked.  Short calls use 4-, 2- or 1-wave
+//    workgroups (16, 8 or 4 tokens; see split_plan).
 //  * per 32-key tile: K and V are staged in LDS (padded row-pair blocks, so
 //    every LDS address is a per-lane base plus an immediate); S^T = K Q^T on
 //    v_mfma_f32_32x32x16_bf16 (A = K from LDS, B = Q^T held in registers for
@@ -637,9 +637,21 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    at 4, 134 unsplit) up to 4096 (166 us against 181; 4500: 204 against
 //    200).  8-token tiles up to 360 tokens (256: 16 us against 17), 16-token
 //    tiles up to 960 (768: 29 us against 33; 1000: 37 against 36).
+//  * few rows over few keys (48 tokens, 1024 keys): a wave's rows and, gated, its
+//    256 gate values a row are a serial chain, so tiles of one wave (4 tokens)
+//    and, over a prefix, chunks of 32 keys up to 8 rows and 64 above (gated, 1
+//    wave / 2 waves and 96 keys / tiles of 256 rows of one head: 4 over 300 8.3 us /
+//    10.2 / 8.9, 8 over 500 9.5 / 11.9 / 12.1, 24 over 256 9.8 / 12.5 / 12.8, 40 8.2 /
+//    9.5 / 9.3, 48 over 500 12.8 / 13.6 / 17.0; only 2 to 12 rows over some 40 keys are
+//    still behind the last, 7.8 / 9.1 / 7.2).  Up to 32 keys there is one chunk; the
+//    plain form then runs unsplit (6 us), the gated one, whose rows would be gated
+//    by a wave or two, still leaves them to the combine (split and combine /
+//    unsplit / one head a workgroup: 1 token 7.0 / 7.3 / 7.2, 8 8.0 / 14.8 / 8.5, 16
+//    8.1 / 15.8 / 10.5, 32 8.2 / 21.0 / 15.0).
 struct SplitPlan {
   unsigned waves, sub, tiles, n_chunks, chunk_keys, ranges, items;   // items: (tile, chunk, KV head) partials
 };
+constexpr unsigned kFewRows = 48, kFewKeys = 1024;
 
 unsigned tile_tokens(unsigned waves) { return waves * kFmRowsPerWave / kGroup; }
 
@@ -651,7 +663,10 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   const bool square = kv_tokens - q_tokens < 256u;
   if (q_tokens > (square ? 4096u : 3072u)) return p;
   const size_t work = (size_t)q_tokens * kv_tokens;
-  if (square)
+  const bool few = q_tokens <= kFewRows && kv_tokens <= kFewKeys;
+  if (few)
+    p.waves = 1u;
+  else if (square)
     p.waves = q_tokens <= 360u ? 2u : q_tokens <= 960u ? 4u : 8u;
   else
     p.waves = work <= 100000u ? 2u : work <= 1400000u ? 4u : 8u;
@@ -666,13 +681,13 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   if (square) {
     n = p.tiles <= 42u ? 4u : p.tiles <= 66u ? 3u : 2u;
   } else {
-    n = std::min(128u / p.tiles, kv_tokens / 96u);
+    n = std::min(128u / p.tiles, kv_tokens / (!few ? 96u : q_tokens <= 8u ? 32u : 64u));
     n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
   }
   const unsigned quantum = kFmKv * p.sub;
   const unsigned chunk = ((kv_tokens + n - 1) / n + quantum - 1) / quantum * quantum;
   n = (kv_tokens + chunk - 1) / chunk;   // after rounding up
-  if (n < 2u) return p;
+  if (n < 2u && !few) return p;
   p.n_chunks = n;
   p.chunk_keys = chunk;
   p.ranges = !square && p.tiles > 1u && p.tiles <= 12u && kv_tokens >= 12000u;
@@ -688,20 +703,20 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
 constexpr size_t kSplitSharedBytes = 66 * 3 * kHkv * kSplitItemBytes;
 
 size_t split_workspace_bytes(const SplitPlan& p) {
-  if (p.n_chunks < 2) return 0;
-  return std::max(kSplitSharedBytes,
-                  (size_t)p.items * (p.waves * p.sub * kFmRowsPerWave) * (kD + 2) * sizeof(float));
+  const size_t exact = (size_t)p.items * (p.waves * p.sub * kFmRowsPerWave) * (kD + 2) * sizeof(float);
+  return p.n_chunks > 1 ? std::max(kSplitSharedBytes, exact) : exact;   // (one chunk: at most 516 KB)
 }
 
 // Whether the call may run with this workspace, and whether it then splits.
-// Without enough of it, calls of up to 2560 tokens are refused and longer ones
-// run unsplit (they do not need the split to fill the GPU).
+// Without enough of it, calls of up to 2560 tokens are refused; longer ones (they
+// do not need the split to fill the GPU) and those of one chunk run unsplit.
 bool split_workspace_ok(unsigned q_tokens, unsigned kv_tokens, const void* workspace,
                         size_t workspace_bytes, bool* split) {
-  const size_t need = split_workspace_bytes(split_plan(q_tokens, kv_tokens));
+  const SplitPlan plan = split_plan(q_tokens, kv_tokens);
+  const size_t need = split_workspace_bytes(plan);
   const bool enough = workspace != nullptr && workspace_bytes >= need;
   *split = need > 0 && enough;
-  return need == 0 || enough || q_tokens > 2560u;
+  return need == 0 || enough || q_tokens > 2560u || plan.n_chunks < 2u;
 }
 
 bool valid_geometry(const void* q, const void* k, const void* v, const float* out,
@@ -721,7 +736,8 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
                           reinterpret_cast<const void*>(fmha_prefill_kernel<2, false>),
                           reinterpret_cast<const void*>(fmha_prefill_kernel<8, true>),
                           reinterpret_cast<const void*>(fmha_prefill_kernel<4, true>),
-                          reinterpret_cast<const void*>(fmha_prefill_kernel<2, true>)}) {
+                          reinterpret_cast<const void*>(fmha_prefill_kernel<2, true>),
+                          reinterpret_cast<const void*>(fmha_prefill_kernel<1, true>)}) {
       const hipError_t e =
           hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kFmLds);
       if (e != hipSuccess) g_fm_attr_status = e;
@@ -740,7 +756,8 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
   const bf16* kb = static_cast<const bf16*>(k);
   const bf16* vb = static_cast<const bf16*>(v);
   const SplitPlan plan = split_plan(q_tokens, kv_tokens);
-  if (plan.n_chunks > 1 && scratch != nullptr) {
+  const bool one_chunk = plan.items > 0 && plan.n_chunks == 1;
+  if (scratch != nullptr && (plan.n_chunks > 1 || (one_chunk && ga.out != nullptr))) {
     SplitArgs sp;
     sp.o = static_cast<float*>(scratch);
     sp.ml = sp.o + (size_t)plan.items * (plan.waves * kFmRowsPerWave) * kD;   // after the O partials
@@ -750,7 +767,8 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
     auto split = plan.sub == 2     ? fmha_prefill_kernel<4, true, false, 2>
                  : plan.waves == 8 ? fmha_prefill_kernel<8, true>
                  : plan.waves == 4 ? fmha_prefill_kernel<4, true>
-                                   : fmha_prefill_kernel<2, true>;
+                 : plan.waves == 2 ? fmha_prefill_kernel<2, true>
+                                   : fmha_prefill_kernel<1, true>;
     hipLaunchKernelGGL(split, dim3(8 * ((plan.tiles * plan.n_chunks + 3) / 4)),
                        dim3(64 * plan.waves * plan.sub), kFmLds * plan.sub, stream, qb, kb, vb, out, q_tokens, kv_tokens,
                        plan.tiles, sp, ga);
@@ -788,8 +806,9 @@ int launch_fmha(const void* q, const void* k, const void* v, float* out,
   }
   // Rows per workgroup without a split: 256 (8 waves) when that gives at
   // least 256 workgroups or the rows extend a cached prefix (long rows); short
-  // square prompts use 128 or 64 rows so they still spread over the CUs.
-  if (2 * tiles(8) >= 256u || kv_tokens > q_tokens) {
+  // square prompts, and rows over one tile of keys (16 over 16: 5.8 us, 7.1 with 8
+  // waves), use 128 or 64 rows so they still spread over the CUs.
+  if (2 * tiles(8) >= 256u || (kv_tokens > q_tokens && !one_chunk)) {
     hipLaunchKernelGGL((fmha_prefill_kernel<8, false>), grid(8), dim3(512), kFmLds, stream,
                        qb, kb, vb, out, q_tokens, kv_tokens, tiles(8), none, ga);
   } else if (2 * tiles(4) >= 256u) {

@@ -126,17 +126,19 @@ def decode_step(q_gate: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
 
 # Up to this many query tokens a split needs its workspace (the C entries refuse
-# the call without) and the calls of a device share one buffer.  Longer ones can
-# run unsplit, so they take memory of their own: they need no eager call before a
-# capture and may run on several streams at once.
+# the call without) and the calls of a device share one buffer.  Longer ones, and
+# those over at most one tile of keys, can run unsplit, so they take memory of
+# their own: they need no eager call before a capture and may run on several
+# streams at once.
 _SHARED_SPLIT_TOKENS = 2560
+_ONE_CHUNK_KEYS = 32
 
 
 def _split_workspace(t: int, s: int, device: torch.device) -> torch.Tensor | None:
     nb = _lib.load(("qwen36_fmha_prefill_workspace_bytes",)).qwen36_fmha_prefill_workspace_bytes(t, s)
     if not nb:
         return None
-    if t > _SHARED_SPLIT_TOKENS:
+    if t > _SHARED_SPLIT_TOKENS or s <= _ONE_CHUNK_KEYS:
         return torch.empty(nb, dtype=torch.uint8, device=device)
     return scratch("fmha_split", nb, device)
 
@@ -166,7 +168,7 @@ def fmha_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         out = torch.empty(t, Q_DIM, dtype=torch.float32, device=q.device)
     require(out, "out", torch.float32, shape=(t, Q_DIM))
     _lib.load(("qwen36_fmha_prefill",))
-    ws = _split_workspace(t, s, q.device)
+    ws = _split_workspace(t, s, q.device) if s > _ONE_CHUNK_KEYS else None
     _lib.call("qwen36_fmha_prefill", ptr(q), ptr(k), ptr(v), ptr(out), t, s, ptr(ws),
               ws.numel() if ws is not None else 0, stream_handle(q.device))
     return out

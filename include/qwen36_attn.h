@@ -59,8 +59,9 @@ int qrt_ck_fmha_release(void);
  * this geometry runs unsplit and workspace may be NULL; also 0 for invalid
  * geometry, which the launch rejects).  Up to 2560 query tokens the size is
  * one for all geometries that split, so one buffer serves them.  From 2561
- * query tokens on the workspace is optional: without enough of it the launch
- * runs unsplit.  Calls that overlap on one workspace race. */
+ * query tokens on, and for up to 32 kv_tokens (where only the gated form uses
+ * it, 516 KB at most), the workspace is optional: without enough of it the
+ * launch runs unsplit.  Calls that overlap on one workspace race. */
 size_t qwen36_fmha_prefill_workspace_bytes(unsigned query_tokens, unsigned kv_tokens);
 int qwen36_fmha_prefill(const void* q, const void* k, const void* v, float* out,
                         unsigned query_tokens, unsigned kv_tokens, void* workspace,

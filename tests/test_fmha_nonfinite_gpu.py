@@ -12,7 +12,7 @@ TOL = 5 * 2.0 ** -8 + 1e-4   # P rounded to bf16 (2^-8 of each at most), |v| bel
 
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("t,s,key", [
-    (33, 33, 1), (300, 300, 40), (900, 900, 700),     # square: 2, 3 and 4 chunks
+    (7, 7, 1), (20, 31, 15), (33, 33, 1), (24, 600, 300), (300, 300, 40), (900, 900, 700),     # square: 2, 3 and 4 chunks
     (2561, 2561, 100), (4096, 4096, 2100),            # split from 2561 tokens on
     (4097, 4097, 100),                                # unsplit
     (3000, 3400, 50), (40, 900, 450), (100, 1000, 3),

@@ -1,4 +1,4 @@
-"""GPU parity of the FMHA's head-packed tiles (8 query heads x 8, 16 or 32
+"""GPU parity of the FMHA's head-packed tiles (8 query heads x 4, 8, 16 or 32
 tokens a tile) and key-range splits at the edges of the tiles and of the
 split rule, against the CPU oracle's SDPA."""
 import pytest
@@ -8,8 +8,8 @@ from oracle import attention_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# fp32 rows against the fp32 oracle: only P is rounded to bf16, a relative
-# 2^-9 of terms p_j v_j that sum to |o| <= max |v| ~ 5
+# fp32 rows against the fp32 oracle: only P is rounded to bf16, by at most 2^-8 of
+# each term p_j v_j, independently (their sum stays below max |v| ~ 5)
 TOL = 5e-3
 TOL_BF16 = 2e-2   # the gated rows' bf16 roundings
 
@@ -88,3 +88,38 @@ def test_long_split_without_workspace_runs_unsplit(gpu):
     assert lib.qwen36_fmha_prefill(*args, 2560, 2560, None, 0, st) == 1
     assert lib.qwen36_fmha_prefill(*args, t, t, None, 0, st) == 0
     assert (out - fmha_prefill(q, k, v)).abs().max().item() <= 2 * TOL
+
+
+@pytest.mark.parametrize("t,s", [
+    (1, 1), (3, 3), (4, 4), (5, 5), (1, 32), (29, 32), (32, 32),       # one chunk
+    (1, 33), (33, 33), (48, 48), (49, 49), (5, 60), (17, 200),         # square
+    (1, 257), (4, 320), (8, 1024), (9, 512), (24, 700), (45, 1000), (48, 1024),   # chunks of 32, 64 keys
+    (48, 1025), (49, 1024)])                                           # 2 waves
+def test_few_rows(gpu, t, s):
+    """Tiles of one wave (4 tokens) and the one chunk of up to 32 keys: rows against
+    64 bits, the gated rows' bits against the gate applied to the plain ones, and the
+    optional workspace of one chunk."""
+    from oracle.attention_bounds import Row
+    from qwen36_attn import _lib
+    from qwen36_attn.full_attention import fmha_prefill, fmha_prefill_gated, output_gate
+    g = torch.Generator().manual_seed(1000 * t + s)
+    q, k, v = (torch.randn(n, h, 256, generator=g).to(torch.bfloat16) for n, h in ((t, 16), (s, 2), (s, 2)))
+    qg = torch.randn(t, 8192, generator=g).to(torch.bfloat16).to(gpu)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    print(f"few rows T={t} S={s}", flush=True)
+    rows, gated = fmha_prefill(qd, kd, vd), fmha_prefill_gated(qd, kd, vd, qg)
+    for r in sorted({0, 3, 4, t // 2, t - 1} & set(range(t))):
+        row = Row(q[r], k[:s - t + r + 1], v[:s - t + r + 1])
+        assert ((rows[r].cpu().double() - row.ref).abs() <= row.tol).all(), r
+    assert torch.equal(gated, output_gate(rows, qg))
+    lib = _lib.load(("qwen36_fmha_prefill", "qwen36_fmha_prefill_gated"))
+    st = torch.cuda.current_stream().cuda_stream
+    out, out16 = torch.empty_like(rows), torch.empty_like(gated)
+    plain = lib.qwen36_fmha_prefill(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(),
+                                    t, s, None, 0, st)
+    fused = lib.qwen36_fmha_prefill_gated(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), qg.data_ptr(),
+                                          8192, out16.data_ptr(), t, s, None, 0, st)
+    torch.cuda.synchronize()
+    assert plain == fused == (0 if s <= 32 else 1)
+    if s <= 32:
+        assert torch.equal(out, rows) and torch.equal(out16, gated)

@@ -12,11 +12,13 @@ def test_one_size_up_to_2560_tokens():
     size = _lib.load(("qwen36_fmha_prefill_workspace_bytes",)).qwen36_fmha_prefill_workspace_bytes
     for t in [*range(1, 2561, 7), 360, 361, 672, 960, 961, 1344, 2048, 2111, 2112, 2113, 2560]:
         for prefix in (0, 1, 255, 256, 300, 1000, 4000, 24000, 65000):
-            if t + prefix > 32:             # (shorter rows have one chunk)
-                assert size(t, t + prefix) in ((0, ONE_SIZE) if t + prefix <= 64 else (ONE_SIZE,))
+            if t + prefix > 32:
+                assert size(t, t + prefix) == ONE_SIZE
+            else:                           # one chunk: tiles of 4 tokens
+                assert size(t, t + prefix) == (t + 3) // 4 * 2 * 32 * 258 * 4
     for t, s in ((2561, 2561), (4096, 4096), (3072, 9000)):
         assert size(t, s) >= ONE_SIZE
-    assert size(4097, 4097) == size(3073, 9000) == size(1, 1) == 0
+    assert size(4097, 4097) == size(3073, 9000) == 0
 
 
 @pytest.mark.gpu
@@ -50,7 +52,7 @@ def _inputs(t, s, gpu, seed):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("t,s", [(2561, 2561), (4096, 4096), (3072, 3400)])
+@pytest.mark.parametrize("t,s", [(1, 32), (32, 32), (2561, 2561), (4096, 4096), (3072, 3400)])
 def test_capture_without_an_eager_call(gpu, t, s, monkeypatch):
     from qwen36_attn import _lib, _tensors
     from qwen36_attn.full_attention import fmha_prefill, fmha_prefill_gated
