@@ -610,7 +610,13 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    32 .. 42 60 us, 16 73, 64 70; 8 over 65000: 33 us at 128, 41 at 64, 50 at
 //    32).  8 waves, whose tiles read K/V least often, from tokens x keys =
 //    1.4 M (256 over 8000: 54 us against 55; 64 over 64000: 86 against 98),
-//    4 waves below (93 over 8000: 34 us against 38), 2 waves below 0.1 M.
+//    4 waves below (93 over 8000: 34 us against 38), 2 waves below 0.2 M
+//    (2 / 4 waves: 32 over 4000 18.8 us / 23.9, 93 over 1000 18.0 / 22.0, over 1500
+//    21.0 / 23.7, over 2050 23.5 / 22.7, 128 over 1000 20.5 / 24.1, over 1400 22.5 / 25.4,
+//    200 over 700 21.4 / 25.1; 200 over 2000, 0.44 M, 28 / 26.8).  Three and more tiles of 2 waves make
+//    at most 192 workgroups (93 over 1500, n = 5 .. 8 21.0 us, 10 22.8; 128 over 1000,
+//    n = 4 20.1, 8 21.9; 64 over 2000, n = 10 19.6, 17 20.9; two tiles, 12 over 9000,
+//    n = 64 18.5, 40 19.5).
 //    Where 8 waves are chosen, pairs of 4-wave halves (kSub = 2) halve the
 //    partials' traffic (62 MB written and read back at 93 over 24000) but read
 //    each key twice as often, so they pay while a half has at most about 1250
@@ -669,7 +675,7 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   else if (square)
     p.waves = q_tokens <= 360u ? 2u : q_tokens <= 960u ? 4u : 8u;
   else
-    p.waves = work <= 100000u ? 2u : work <= 1400000u ? 4u : 8u;
+    p.waves = work <= 200000u ? 2u : work <= 1400000u ? 4u : 8u;
   const unsigned pairs = (q_tokens + tile_tokens(4u) - 1) / tile_tokens(4u);
   if (!square && p.waves == 8u && pairs >= 6u && pairs <= 42u && 128u / pairs * pairs >= 115u &&
       kv_tokens <= 32768u && (size_t)pairs * kv_tokens <= 1250u * 256u) {
@@ -681,7 +687,8 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
   if (square) {
     n = p.tiles <= 42u ? 4u : p.tiles <= 66u ? 3u : 2u;
   } else {
-    n = std::min(128u / p.tiles, kv_tokens / (!few ? 96u : q_tokens <= 8u ? 32u : 64u));
+    n = std::min((p.waves == 2u && p.tiles > 2u ? 96u : 128u) / p.tiles,
+                 kv_tokens / (!few ? 96u : q_tokens <= 8u ? 32u : 64u));
     n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
   }
   const unsigned quantum = kFmKv * p.sub;

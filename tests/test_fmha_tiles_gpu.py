@@ -16,7 +16,8 @@ TOL_BF16 = 2e-2   # the gated rows' bf16 roundings
 
 @pytest.mark.parametrize("t,s", [
     (8, 8), (9, 9), (33, 33),                    # one chunk (unsplit) and its first split
-    (8, 12000), (9, 12000), (13, 7700),          # 2 / 4 waves, one tile
+    (8, 12000), (9, 12000), (13, 7700),          # 2 waves, one and two tiles
+    (26, 7692), (26, 7693), (93, 1593),          # 2 / 4 waves; 12 tiles of 2 waves
     (3, 60003), (64, 30064),                     # 128 chunks; 8 waves
     (32, 24032), (33, 24033), (93, 24093),       # full and one-token last tiles
     (360, 360), (361, 361), (960, 960), (961, 961), (1345, 1345), (2113, 2113),
