@@ -636,7 +636,11 @@ hipError_t g_fm_attr_status = hipSuccess;
 //    256 over 8000 52.1 / 51.2, 1000 over 4000 91 / 85; short: 93 over 2000 26.1 /
 //    23.9).
 //    Up to 3072 rows two chunks still win (2500 over 4000: 219 us against
-//    299 unsplit; 3500: 339 against 325).
+//    299 unsplit; 3500: 339 against 325).  Where the later chunks of the first tiles
+//    hold no key, three chunks may still be at most one workgroup per CU and take
+//    the place of two (1400 over 1000 65.5 us against 74.1, 1500 over 1500 77.2 /
+//    83.3, 1900 over 256 64.2 / 69.3; with more: 2048 over 256, 136, 79.5 / 74.1, 1900
+//    over 1000, 150, 90.4 / 88.3; 1700 over 1000, 136, would gain, 75.8 / 80.4).
 //  * square prompts: later tiles hold more chunks, 2 tiles (n + 1) / 2 in
 //    all, again about one per CU: n = 4 up to 42 tiles, 3 up to 66, then 2
 //    (2048 tokens: 63 us at n = 3, 68 at 2, 86 at 4; 3072: 105 us at 2, 120
@@ -692,7 +696,17 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
     n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
   }
   const unsigned quantum = kFmKv * p.sub;
-  const unsigned chunk = ((kv_tokens + n - 1) / n + quantum - 1) / quantum * quantum;
+  auto chunk_of = [&](unsigned chunks) {
+    return ((kv_tokens + chunks - 1) / chunks + quantum - 1) / quantum * quantum;
+  };
+  if (!square && n == 2u) {
+    unsigned live = 0;   // (tile, chunk) items of three chunks that hold a key
+    for (unsigned i = 1; i <= p.tiles; ++i)
+      live += (std::min(i * tile_tokens(p.waves), q_tokens) + kv_tokens - q_tokens + chunk_of(3u) - 1) /
+              chunk_of(3u);
+    if (live <= 128u) n = 3u;
+  }
+  const unsigned chunk = chunk_of(n);
   n = (kv_tokens + chunk - 1) / chunk;   // after rounding up
   if (n < 2u && !few) return p;
   p.n_chunks = n;

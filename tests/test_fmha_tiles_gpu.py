@@ -23,6 +23,7 @@ TOL_BF16 = 2e-2   # the gated rows' bf16 roundings
     (360, 360), (361, 361), (960, 960), (961, 961), (1345, 1345), (2113, 2113),
     (4096, 4096), (4097, 4097),                  # last split and first unsplit length
     (3072, 3400), (3073, 3400),                  # the same over a prefix
+    (1376, 2376), (1900, 2156), (1900, 2400),    # three chunks in place of two; two
 ])
 def test_tile_and_split_edges(gpu, t, s):
     from qwen36_attn.full_attention import fmha_prefill, fmha_prefill_gated, output_gate
