@@ -692,7 +692,9 @@ SplitPlan split_plan(unsigned q_tokens, unsigned kv_tokens) {
     n = p.tiles <= 42u ? 4u : p.tiles <= 66u ? 3u : 2u;
   } else {
     n = std::min((p.waves == 2u && p.tiles > 2u ? 96u : 128u) / p.tiles,
-                 kv_tokens / (!few ? 96u : q_tokens <= 8u ? 32u : 64u));
+                 !few             ? kv_tokens / 96u
+                 : q_tokens <= 8u ? (kv_tokens + 31u) / 32u
+                                  : (kv_tokens + 63u) / 64u);
     n = std::max(2u, std::min(n, (unsigned)kCombineMaxChunks));
   }
   const unsigned quantum = kFmKv * p.sub;
